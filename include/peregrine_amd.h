@@ -304,6 +304,17 @@ int32_t pga_wall_flux(const pga_case *c, int32_t axis, int32_t side, const pga_w
                       int32_t ng, pga_view Q, pga_view state, pga_view trstate, pga_view xcc, pga_view xf, pga_view S,
                       pga_view F, void *stream);
 
+/* Both hooks for a block's nwall walls (0 to 6, each face once) in one launch: wall n on face sides[n]
+ * of axes[n] with walls[n] (null walls: adiabatic slip walls), its faces' area vectors S[n], fluxes
+ * F[n] and (a viscous case) centres xf[n]. The values are the single calls'. */
+int32_t pga_wall_mirrors(const pga_case *c, int32_t nwall, const int32_t *axes, const int32_t *sides,
+                         const pga_wall *walls, const int32_t *ncell, int32_t ng, pga_view Q, pga_view state,
+                         const pga_view *S, void *stream);
+int32_t pga_wall_fluxes(const pga_case *c, int32_t nwall, const int32_t *axes, const int32_t *sides,
+                        const pga_wall *walls, const int32_t *ncell, int32_t ng, pga_view Q, pga_view state,
+                        pga_view trstate, pga_view xcc, const pga_view *xf, const pga_view *S, const pga_view *F,
+                        void *stream);
+
 /* The CFL reduction over the cells of `box`: out[0..2] (device memory) receive the largest
  * acoustic c sqrt(sum 1/d^2), convective sum |u . n| / d and combined (their sum) inverse time
  * scales, each folded by fmax from -inf; d the cell's lengths (dijk, infinite along an axis one

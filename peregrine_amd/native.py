@@ -115,6 +115,10 @@ SIGNATURES = {
     "pga_wall_mirror": (_i32, [C.c_void_p, _i32, _i32, C.c_void_p, _ip, _i32, View, View, View, C.c_void_p]),
     "pga_wall_flux": (_i32, [C.c_void_p, _i32, _i32, C.c_void_p, _ip, _i32, View, View, View, View, View, View, View,
                              C.c_void_p]),
+    "pga_wall_mirrors": (_i32, [C.c_void_p, _i32, _ip, _ip, C.POINTER(Wall), _ip, _i32, View, View, C.POINTER(View),
+                                C.c_void_p]),
+    "pga_wall_fluxes": (_i32, [C.c_void_p, _i32, _ip, _ip, C.POINTER(Wall), _ip, _i32, View, View, View, View,
+                               C.POINTER(View), C.POINTER(View), C.POINTER(View), C.c_void_p]),
     "pga_cflmax_worksize": (C.c_int64, [Box]),
     "pga_substep_listsize": (C.c_int64, [C.POINTER(SubstepOpts), Box]),
     "pga_substep": (_i32, [C.c_void_p, C.POINTER(SubstepOpts), View, View, View, _i32, C.c_void_p, C.c_int64,

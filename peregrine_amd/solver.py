@@ -533,20 +533,29 @@ class Solver:
                     self._call("pga_diffflux", self.case.handle, a, self.sim.alpha, Qv, st, blk.trstate.view(),
                                blk.hsp.view(), blk.grads.view(), blk.xcc.view(), blk.xf[a].view(), S.view(),
                                F.view(), boxes[a])
-        for axis, side, wall in blk.walls:
-            S, F = (blk.iS, blk.jS, blk.kS)[axis], (blk.iF, blk.jF, blk.kF)[axis]
+        if blk.walls:
+            n, axes, head = self._walls(blk)
             visc = self.sim.viscous
-            self._call("pga_wall_flux", self.case.handle, axis, side, ctypes.byref(wall), native.ints(blk.ncell),
-                       self.ng, Qv, st, blk.trstate.view() if visc else native.View(), blk.xcc.view(),
-                       blk.xf[axis].view() if visc else native.View(), S.view(), F.view())
+            S, F, xf = ((native.View * n)(*[arr[a].view() for a in axes]) for arr in (
+                (blk.iS, blk.jS, blk.kS), (blk.iF, blk.jF, blk.kF), blk.xf if visc else (blk.iF, blk.jF, blk.kF)))
+            self._call("pga_wall_fluxes", *head, Qv, st, blk.trstate.view() if visc else native.View(),
+                       blk.xcc.view(), xf if visc else None, S, F)
+
+    def _walls(self, blk):
+        """(walls, their axes, the leading arguments both wall hooks take) of a block."""
+        axes, sides, walls = zip(*blk.walls)
+        n = len(axes)
+        return n, axes, (self.case.handle, n, native.ints(axes), native.ints(sides), (native.Wall * n)(*walls),
+                         native.ints(blk.ncell), self.ng)
 
     def wall_halos(self, Q):
-        """Each wall's halo as the interior's mirror image (the preadvflux hook)."""
+        """Each wall's halo as the interior's mirror image (the preadvflux hook), a block's in one
+        launch."""
         for blk in self.blocks:
-            for axis, side, wall in blk.walls:
-                S = (blk.iS, blk.jS, blk.kS)[axis]
-                self._call("pga_wall_mirror", self.case.handle, axis, side, ctypes.byref(wall), native.ints(blk.ncell),
-                           self.ng, blk.regs[Q].view(), blk.state.view(), S.view())
+            if blk.walls:
+                n, axes, head = self._walls(blk)
+                S = (native.View * n)(*[(blk.iS, blk.jS, blk.kS)[a].view() for a in axes])
+                self._call("pga_wall_mirrors", *head, blk.regs[Q].view(), blk.state.view(), S)
 
     def prerhs(self, Q, dQ=None):
         self.exchange(Q)
