@@ -139,6 +139,14 @@ struct View {
   __device__ __forceinline__ double &at(int64_t o, int c) const {
     return *reinterpret_cast<double *>(reinterpret_cast<char *>(d + c * sc) + (uint32_t)((uint64_t)o << 3));
   }
+  // at() for a run of components of one cell, b its byte offset in a plane: each access takes the plane's
+  // scalar base and b as it is. The compiler is kept from seeing that b is the same throughout, or it adds
+  // the first base to it and the others to that, 64-bit vector additions and registers for each
+  __device__ __forceinline__ double &run(uint32_t &b, int c) const {
+    asm("" : "+v"(b));
+    return *reinterpret_cast<double *>(reinterpret_cast<char *>(d + c * sc) + b);
+  }
+  __device__ __forceinline__ static uint32_t bytes(int64_t o) { return (uint32_t)((uint64_t)o << 3); }
 };
 
 __host__ inline View view(const pga_view &v) { return View{v.data, v.sj, v.sk, v.sc}; }
@@ -166,6 +174,20 @@ __host__ inline Box3 box3(const pga_box &b) {
 
 __host__ inline dim3 grid_of(const Box3 &b) {
   return dim3((b.e0 + TI - 1) / TI, (b.e1 + TJ - 1) / TJ, b.e2);
+}
+
+// n / d for n < 2^31 by a multiply-high and a shift set up on the host (Granlund and Montgomery, Division
+// by invariant integers using multiplication, PLDI 1994, Fig. 4.1): a division in the kernel is some
+// twenty instructions of every lane
+struct FastDiv {
+  unsigned d, m, s;
+  __device__ __forceinline__ unsigned operator()(unsigned n) const { return (__umulhi(m, n) + n) >> s; }
+};
+
+__host__ inline FastDiv fast_div(unsigned d) {
+  unsigned s = 0;
+  while ((uint64_t(1) << s) < d) s++;
+  return FastDiv{d, (unsigned)((((uint64_t(1) << s) - d) << 32) / d + 1), s};
 }
 
 // Flat launches: 256-thread blocks over the box's cells in i-fastest order, so a row
@@ -219,14 +241,15 @@ __device__ __forceinline__ T *opaque(T *p) {
   return p;
 }
 
-// the cell of a flat tile t of box b, false past the box
+// the cell of a flat tile t of box b, false past the box (a box lies in a plane of at most 2^29
+// doubles, so its cells count in 32 bits)
 __device__ __forceinline__ bool flat_at(const Box3 &b, int64_t t, int &i, int &j, int &k) {
-  const int64_t c = t * FLAT + threadIdx.x;
-  const int64_t row = c / b.e0;
-  i = b.s0 + (int)(c - row * b.e0);
-  j = b.s1 + (int)(row % b.e1);
-  k = b.s2 + (int)(row / b.e1);
-  return row < (int64_t)b.e1 * b.e2;
+  const unsigned c = (unsigned)t * FLAT + threadIdx.x;
+  const unsigned row = c / (unsigned)b.e0;
+  i = b.s0 + (int)(c - row * (unsigned)b.e0);
+  j = b.s1 + (int)(row % (unsigned)b.e1);
+  k = b.s2 + (int)(row / (unsigned)b.e1);
+  return row < (unsigned)b.e1 * (unsigned)b.e2;
 }
 
 // the cell a thread takes, false when the block overhangs the box
@@ -318,6 +341,42 @@ __device__ __forceinline__ double elog(double x) {
   const double finite = fabs(r1) < 0.03125 ? series : table;
   const double limit = x == 0.0 ? -__builtin_huge_val() : x > 0.0 ? x : __builtin_nan("");
   return x > 0.0 && x <= 1.7976931348623157e308 ? finite : limit;
+}
+
+// elog's table path alone, for a positive normal x no nearer to 1 than 1/32
+__device__ __forceinline__ double elog_table(double x) {
+#pragma clang fp contract(off)
+  const long long bits = __double_as_longlong(x);
+  const int e = (int)((bits >> 52) & 0x7ff) - 1023;
+  const int k = (int)((bits >> 45) & 127);
+  const double m = __longlong_as_double((bits & 0x000fffffffffffffLL) | 0x3ff0000000000000LL);
+  const double r = fma(m, ELOG_RCP[k], -1.0);
+  double q = 1.0 / 7.0;
+  q = fma(q, r, -1.0 / 6.0);
+  q = fma(q, r, 0.2);
+  q = fma(q, r, -0.25);
+  q = fma(q, r, 1.0 / 3.0);
+  q = fma(q, r, -0.5);
+  const double p = (r * r) * q;
+  const double hi = e * PGA_ELOG_LN2HI + ELOG_LHI[k];
+  const double lo = e * PGA_ELOG_LN2LO + ELOG_LLO[k];
+  return hi + (r + (p + lo));
+}
+
+__device__ __forceinline__ bool elog_far(double x) {
+  return x >= 2.2250738585072014e-308 && x <= 1.7976931348623157e308 && fabs(x - 1.0) >= 0.03125;
+}
+
+// elog of two temperatures, elog's bits: the table path, which any gas's T takes, and elog whole only for
+// lanes where either T is near 1 or no positive normal number (skipped by a wave that has none; the series
+// and the limits are half of elog's instructions)
+__device__ __forceinline__ void elog2(double xa, double xb, double &la, double &lb) {
+  la = elog_table(xa);
+  lb = elog_table(xb);
+  if (!(elog_far(xa) && elog_far(xb))) {
+    la = elog(xa);
+    lb = elog(xb);
+  }
 }
 
 // ln(1 + x) through elog: u = 1 + x rounded, then the first-order correction for that rounding,

@@ -139,10 +139,10 @@ __device__ __forceinline__ void mixmom2(const Gas<NS> &g, const YA &Ya, const YB
 
 // caloric/tdepcp/kernels/caloric.mako:4-15: cp and h per mass at T, h's coefficients
 // built in the same descent as hcoeff[m] = cpcoeff[m] - (m + 1) hcoeff[m + 1]
+// (u = ln T)
 template <class M>
-__device__ __forceinline__ void ideal_cph(const M &m, double T, double &cp, double &h) {
+__device__ __forceinline__ void ideal_cph(const M &m, double T, double u, double &cp, double &h) {
 #pragma clang fp contract(off)
-  const double u = elog(T);
   double cpv = 0.0, hv = 0.0, hc = 0.0;
 #pragma unroll
   for (int t = NT - 1; t >= 0; t--) {
@@ -152,6 +152,11 @@ __device__ __forceinline__ void ideal_cph(const M &m, double T, double &cp, doub
   }
   cp = cpv;
   h = fma(hv, T, m.h298);
+}
+
+template <class M>
+__device__ __forceinline__ void ideal_cph(const M &m, double T, double &cp, double &h) {
+  ideal_cph(m, T, elog(T), cp, h);
 }
 
 // ---------------------------------------------------------------------------
@@ -397,10 +402,11 @@ __device__ __forceinline__ void fromrhoE(const Gas<NS> &g, const MixMom<NS, EOS>
   }
 }
 
-// (p, T) -> state: cpg eos.mako:17-27, tpg eos.mako:22-33, real gas eos/realgas/kernels/eos.mako:137-155
-template <int NS, int EOS, class YF>
+// (p, T) -> state: cpg eos.mako:17-27, tpg eos.mako:22-33, real gas eos/realgas/kernels/eos.mako:137-155;
+// lnT() gives elog(T), of which a thermally perfect gas takes one
+template <int NS, int EOS, class YF, class LF>
 __device__ __forceinline__ void frompT(const Gas<NS> &g, const MixMom<NS, EOS> &m, const YF &Y, double p, double T,
-                                       EosState &s) {
+                                       const LF &lnT, EosState &s) {
 #pragma clang fp contract(off)
   if constexpr (EOS == EOS_REAL) {
     Cubic c;
@@ -433,7 +439,7 @@ __device__ __forceinline__ void frompT(const Gas<NS> &g, const MixMom<NS, EOS> &
       s.gamma = m.cp / cv;
     } else {
       double cp, h;
-      ideal_cph(m, T, cp, h);
+      ideal_cph(m, T, lnT(), cp, h);
       s.e = h - m.R * T;
       s.cp = cp;
       s.gamma = cp / (cp - m.R);
@@ -441,6 +447,12 @@ __device__ __forceinline__ void frompT(const Gas<NS> &g, const MixMom<NS, EOS> &
     s.c = sqrt(s.gamma * m.R * T);
     s.Z = 1.0;
   }
+}
+
+template <int NS, int EOS, class YF>
+__device__ __forceinline__ void frompT(const Gas<NS> &g, const MixMom<NS, EOS> &m, const YF &Y, double p, double T,
+                                       EosState &s) {
+  frompT<NS, EOS>(g, m, Y, p, T, [&]() { return elog(T); }, s);
 }
 
 template <int EOS>

@@ -23,98 +23,107 @@ struct FaceState {
 
 enum { LIM_NONE = 0, LIM_KOREN = 1, LIM_MINMOD = 2, LIM_MC = 3, LIM_SUPERBEE = 4, LIM_VANLEER = 5 };
 
-// b phi(a / b), b > 0, without the ratio (recon/{koren,minmod,mc,superbee,vanleer}.mako)
+// half of b phi(a / b), b >= 0, without the ratio (recon/{koren,minmod,mc,superbee,vanleer}.mako). Koren's
+// min(min(2a, (2b + a) / 3), 2b) halved is min(min(a, ((2b + a) / 3) / 2), b): halving is exact, and so is
+// 2b inside the fused add
 template <int LIM>
-__device__ __forceinline__ double limit(double a, double b) {
+__device__ __forceinline__ double half_limit(double a, double b) {
 #pragma clang fp contract(off)
-  if constexpr (LIM == LIM_KOREN) return fmax(0.0, fmin(fmin(2.0 * a, (2.0 * b + a) * (1.0 / 3.0)), 2.0 * b));
-  if constexpr (LIM == LIM_MINMOD) return fmax(0.0, fmin(b, a));
-  if constexpr (LIM == LIM_MC) return fmax(0.0, fmin(fmin(2.0 * a, (b + a) * 0.5), 2.0 * b));
-  if constexpr (LIM == LIM_SUPERBEE) return fmax(0.0, fmax(fmin(2.0 * a, b), fmin(a, 2.0 * b)));
-  return (a + fabs(a)) * b / (b + fabs(a));
+  if constexpr (LIM == LIM_KOREN) return fmax(0.0, fmin(fmin(a, 0.5 * (fma(2.0, b, a) * (1.0 / 3.0))), b));
+  if constexpr (LIM == LIM_MINMOD) return fmax(0.0, 0.5 * fmin(b, a));
+  if constexpr (LIM == LIM_MC) return fmax(0.0, fmin(fmin(a, 0.5 * ((b + a) * 0.5)), b));
+  if constexpr (LIM == LIM_SUPERBEE) return 0.5 * fmax(0.0, fmax(fmin(2.0 * a, b), fmin(a, 2.0 * b)));
+  return 0.5 * ((a + fabs(a)) * b / (b + fabs(a)));
 }
 
-// recon/muscl.mako:5-13: the limited slope across the face carried to dp's sign and back; zero
-// where dp is. Evaluated on every lane and selected, so the 26 slopes of a face stay one basic
-// block the scheduler can interleave (a branch per slope would fence each one off)
+// recon/muscl.mako:5-13 for both sides of a face: L = vL + phi(vL - vLL, dp) / 2 and R = vR - phi(vRR - vR,
+// dp) / 2, dp = vR - vL, phi the limited slope carried to dp's sign and back. The sign is a factor +-1 whose
+// product is exact, so it is folded into the last add. A zero dp gives a zero slope by itself (b = 0), but
+// van Leer's, which would divide by b. Evaluated on every lane and selected, so the 26 slopes of a face
+// stay one basic block the scheduler can interleave. 21 instructions a pair where the two slopes apart,
+// with their scalings and a select each, were 33: 170 of the 1230 a nine-species face takes
 template <int LIM>
-__device__ __forceinline__ double phi(double dm, double dp) {
+__device__ __forceinline__ void limited_sides(double vLL, double vL, double vR, double vRR, double &l, double &r) {
 #pragma clang fp contract(off)
-  const double s = copysign(1.0, dp);
-  const double p = s * limit<LIM>(s * dm, fabs(dp));
-  return dp != 0.0 ? p : 0.0;
-}
-
-template <int LIM>
-__device__ __forceinline__ double left_of(double vLL, double vL, double vR) {
-#pragma clang fp contract(off)
-  return vL + 0.5 * phi<LIM>(vL - vLL, vR - vL);
-}
-
-template <int LIM>
-__device__ __forceinline__ double right_of(double vL, double vR, double vRR) {
-#pragma clang fp contract(off)
-  return vR - 0.5 * phi<LIM>(vRR - vR, vR - vL);
-}
-
-// the face's sides: recon/constant.mako:3-18 (the two cells as they are) or
-// recon/muscl.mako:15-51 (p, T, Y and velocity limited, each side closed by the eos from p, T, Y);
-// o is the offset of the face's right cell R, d the stride along the axis
-// evaluated with one rounding per operation: the sides' p and T feed the EOS's ill-conditioned
-// ln T polynomials, where a last-bit change in T moves e by 1e-11 of itself
-template <int NS, int EOS, int RECON, int LIM>
-__device__ __forceinline__ void face_sides(const Gas<NS> &g, const View &Q, const View &st, int64_t o, int64_t d,
-                                           FaceState<NS> &L, FaceState<NS> &R) {
-#pragma clang fp contract(off)
-  if constexpr (RECON == RECON_CONSTANT) {
-    const int64_t oL = o - d;
-    load_state(st, oL, L.s);
-    load_state(st, o, R.s);
-    const double rL = Q.at(oL, 0), rR = Q.at(o, 0);
-    L.u = Q.at(oL, 1) / rL;
-    L.v = Q.at(oL, 2) / rL;
-    L.w = Q.at(oL, 3) / rL;
-    R.u = Q.at(o, 1) / rR;
-    R.v = Q.at(o, 2) / rR;
-    R.w = Q.at(o, 3) / rR;
-#pragma unroll
-    for (int n = 0; n < NS - 1; n++) {
-      L.Y[n] = Q.at(oL, 5 + n) / rL;
-      R.Y[n] = Q.at(o, 5 + n) / rR;
-    }
-  } else {
-    const int64_t oLL = o - 2 * d, oL = o - d, oRR = o + d;
-    const double ri0 = st.at(oLL, 2), ri1 = st.at(oL, 2), ri2 = st.at(o, 2), ri3 = st.at(oRR, 2);
-    const double p0 = st.at(oLL, 0), p1 = st.at(oL, 0), p2 = st.at(o, 0), p3 = st.at(oRR, 0);
-    const double T0 = st.at(oLL, 1), T1 = st.at(oL, 1), T2 = st.at(o, 1), T3 = st.at(oRR, 1);
-    const double pL = left_of<LIM>(p0, p1, p2), pR = right_of<LIM>(p1, p2, p3);
-    const double TL = left_of<LIM>(T0, T1, T2), TR = right_of<LIM>(T1, T2, T3);
-#pragma unroll
-    for (int n = 0; n < NS - 1; n++) {
-      const double y0 = Q.at(oLL, 5 + n) * ri0, y1 = Q.at(oL, 5 + n) * ri1;
-      const double y2 = Q.at(o, 5 + n) * ri2, y3 = Q.at(oRR, 5 + n) * ri3;
-      L.Y[n] = left_of<LIM>(y0, y1, y2);
-      R.Y[n] = right_of<LIM>(y1, y2, y3);
-    }
-    MixMom<NS, EOS> mL, mR;
-    mixmom2<NS, EOS>(g, [&](int n) { return L.Y[n]; }, [&](int n) { return R.Y[n]; }, mL, mR);
-    frompT<NS, EOS>(g, mL, [&](int n) { return L.Y[n]; }, pL, TL, L.s);
-    double vel[3][4];
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      vel[c][0] = Q.at(oLL, 1 + c) * ri0;
-      vel[c][1] = Q.at(oL, 1 + c) * ri1;
-      vel[c][2] = Q.at(o, 1 + c) * ri2;
-      vel[c][3] = Q.at(oRR, 1 + c) * ri3;
-    }
-    L.u = left_of<LIM>(vel[0][0], vel[0][1], vel[0][2]);
-    L.v = left_of<LIM>(vel[1][0], vel[1][1], vel[1][2]);
-    L.w = left_of<LIM>(vel[2][0], vel[2][1], vel[2][2]);
-    frompT<NS, EOS>(g, mR, [&](int n) { return R.Y[n]; }, pR, TR, R.s);
-    R.u = right_of<LIM>(vel[0][1], vel[0][2], vel[0][3]);
-    R.v = right_of<LIM>(vel[1][1], vel[1][2], vel[1][3]);
-    R.w = right_of<LIM>(vel[2][1], vel[2][2], vel[2][3]);
+  const double dp = vR - vL, s = copysign(1.0, dp), b = fabs(dp);
+  double hl = half_limit<LIM>(s * (vL - vLL), b), hr = half_limit<LIM>(s * (vRR - vR), b);
+  if constexpr (LIM == LIM_VANLEER) {
+    hl = dp != 0.0 ? hl : 0.0;
+    hr = dp != 0.0 ? hr : 0.0;
   }
+  l = fma(s, hl, vL);
+  r = fma(-s, hr, vR);
+}
+
+// the face's sides from the two cells as they are (recon/constant.mako:3-18); o is the offset of the
+// face's right cell R, d the stride along the axis
+template <int NS>
+__device__ __forceinline__ void constant_sides(const View &Q, const View &st, int64_t o, int64_t d, FaceState<NS> &L,
+                                               FaceState<NS> &R) {
+#pragma clang fp contract(off)
+  const int64_t oL = o - d;
+  load_state(st, oL, L.s);
+  load_state(st, o, R.s);
+  const double rL = Q.at(oL, 0), rR = Q.at(o, 0);
+  L.u = Q.at(oL, 1) / rL;
+  L.v = Q.at(oL, 2) / rL;
+  L.w = Q.at(oL, 3) / rL;
+  R.u = Q.at(o, 1) / rR;
+  R.v = Q.at(o, 2) / rR;
+  R.w = Q.at(o, 3) / rR;
+#pragma unroll
+  for (int n = 0; n < NS - 1; n++) {
+    L.Y[n] = Q.at(oL, 5 + n) / rL;
+    R.Y[n] = Q.at(o, 5 + n) / rR;
+  }
+}
+
+// the primitives MUSCL limits, by number: p, T, the velocity, the carried mass fractions
+enum { PRIM_P = 0, PRIM_T = 1, PRIM_U = 2, PRIM_Y = 5 };
+
+// the primitives of a face's four cells LL, L, R, RR (m = 0..3), read from the cell arrays
+template <int NS>
+struct ArrayStencil {
+  const View &Q, &st;
+  int64_t o, d;
+  double ri[4];
+  __device__ __forceinline__ ArrayStencil(const View &Q_, const View &st_, int64_t o_, int64_t d_)
+      : Q(Q_), st(st_), o(o_), d(d_) {
+#pragma unroll
+    for (int m = 0; m < 4; m++) ri[m] = st.at(o + (m - 2) * d, 2);
+  }
+  __device__ __forceinline__ double operator()(int v, int m) const {
+#pragma clang fp contract(off)
+    const int64_t om = o + (m - 2) * d;
+    if (v < PRIM_U) return st.at(om, v);
+    return Q.at(om, v < PRIM_Y ? v - 1 : v) * ri[m];
+  }
+};
+
+// the face's sides by MUSCL (recon/muscl.mako:15-51): p, T, Y and the velocity limited, each side closed
+// by the eos from p, T, Y. Evaluated with one rounding per operation: the sides' p and T feed the EOS's
+// ill-conditioned ln T polynomials, where a last-bit change in T moves e by 1e-11 of itself
+template <int NS, int EOS, int LIM, class SRC>
+__device__ __forceinline__ void muscl_sides(const Gas<NS> &g, const SRC &x, FaceState<NS> &L, FaceState<NS> &R) {
+#pragma clang fp contract(off)
+  const auto sides = [&](int v, double &l, double &r) {
+    limited_sides<LIM>(x(v, 0), x(v, 1), x(v, 2), x(v, 3), l, r);
+  };
+  // T and its logarithms first: the species' constants, which the branch in elog2 would otherwise keep in
+  // scalar registers across it, are not loaded yet
+  double pL, pR, TL, TR, uL = 0.0, uR = 0.0;
+  sides(PRIM_T, TL, TR);
+  if constexpr (EOS == EOS_TPG) elog2(TL, TR, uL, uR);
+  sides(PRIM_P, pL, pR);
+#pragma unroll
+  for (int n = 0; n < NS - 1; n++) sides(PRIM_Y + n, L.Y[n], R.Y[n]);
+  MixMom<NS, EOS> mL, mR;
+  mixmom2<NS, EOS>(g, [&](int n) { return L.Y[n]; }, [&](int n) { return R.Y[n]; }, mL, mR);
+  frompT<NS, EOS>(g, mL, [&](int n) { return L.Y[n]; }, pL, TL, [&]() { return uL; }, L.s);
+  sides(PRIM_U, L.u, R.u);
+  sides(PRIM_U + 1, L.v, R.v);
+  sides(PRIM_U + 2, L.w, R.w);
+  frompT<NS, EOS>(g, mR, [&](int n) { return R.Y[n]; }, pR, TR, [&]() { return uR; }, R.s);
 }
 
 // function/kepaec.mako:2-20 (Shima et al. 2021): arithmetic means, the harmonic mean of cv T
@@ -217,6 +226,22 @@ __device__ __forceinline__ void flux_function(const FaceState<NS> &L, const Face
     rusanov<NS>(L, R, S, F);
 }
 
+// the face's area vector, read by this face alone
+__device__ __forceinline__ void load_area(const View &S, int i, int j, int k, double (&Sv)[3]) {
+  uint32_t b = View::bytes(S.off(i, j, k));
+#pragma unroll
+  for (int d = 0; d < 3; d++) Sv[d] = __builtin_nontemporal_load(&S.run(b, d));
+}
+
+// The face's flux stored past the caches: a face value is written once and read back by the stage from HBM
+// in any case, and the stencil's Q and state keep L2 (5% on the 128^3 step's faces)
+template <int NS>
+__device__ __forceinline__ void store_flux(const View &F, int i, int j, int k, const double (&Fv)[NS + 4]) {
+  uint32_t b = View::bytes(F.off(i, j, k));
+#pragma unroll
+  for (int l = 0; l < NS + 4; l++) __builtin_nontemporal_store(Fv[l], &F.run(b, l));
+}
+
 // the face (i, j, k) of `axis` (between cells k - 1 and k along it): its sides, its flux into Fv
 template <int NS, int EOS, int RECON, int PRIMARY, int LIM>
 __device__ __forceinline__ void flux_at(const double *__restrict__ K, int axis, const View &Q, const View &st,
@@ -225,11 +250,12 @@ __device__ __forceinline__ void flux_at(const double *__restrict__ K, int axis, 
   const int64_t o = Q.off(i, j, k);
   const int64_t d = axis == 0 ? 1 : axis == 1 ? Q.sj : Q.sk;
   FaceState<NS> L, R;
-  face_sides<NS, EOS, RECON, LIM>(g, Q, st, o, d, L, R);
-  // the face's area vector is read by this face alone
-  const int64_t of = S.off(i, j, k);
-  const double Sv[3] = {__builtin_nontemporal_load(&S.at(of, 0)), __builtin_nontemporal_load(&S.at(of, 1)),
-                        __builtin_nontemporal_load(&S.at(of, 2))};
+  if constexpr (RECON == RECON_CONSTANT)
+    constant_sides<NS>(Q, st, o, d, L, R);
+  else
+    muscl_sides<NS, EOS, LIM>(g, ArrayStencil<NS>(Q, st, o, d), L, R);
+  double Sv[3];
+  load_area(S, i, j, k, Sv);
   flux_function<NS, PRIMARY>(L, R, Sv, Fv);
 }
 
@@ -239,9 +265,167 @@ __device__ __forceinline__ void flux_face(const double *__restrict__ K, int axis
                                           const View &S, const View &F, int i, int j, int k) {
   double Fv[NS + 4];
   flux_at<NS, EOS, RECON, PRIMARY, LIM>(K, axis, Q, st, S, i, j, k, Fv);
-  const int64_t oF = F.off(i, j, k);
+  store_flux<NS>(F, i, j, k, Fv);
+}
+
+// ---------------------------------------------------------------------------
+// MUSCL faces by tiles: the workgroup's 256 faces read their cells' primitives from LDS, where each cell
+// of the tile is put once. A face of its own reads 56 values of the cell arrays for nine species, more than
+// registers hold in flight beside the sides and their EOS, so it waited on memory several times over at
+// three waves a SIMD. Staged, a thread has the 14 loads of a cell or two in flight at once and waits once,
+// the velocities and mass fractions are divided out once a cell and not four times, and the stencils'
+// reads are LDS's: the faces of the reacting 128^3 block went from 440 to 409 us a launch, 382 with the
+// limiter's and the indexes' shorter forms below, which is 4.2 TB/s of the 4.8 a plain copy reaches here
+// (four waves a SIMD in place of three then change nothing). The cubic real gas is bound by its roots and
+// logarithms, not by these loads: staged, the faces of the 256 x 128 x 64 layer took 732 us against 686,
+// so it reads its stencils from the arrays.
+//
+// i faces: nf consecutive faces of the box's rows, a row's run of them with its three cells more. j and k
+// faces: wi faces along i by 256 / wi along the axis, with three planes of cells more. A cell's values lie
+// side by side (an odd number of doubles, so the lanes' slots spread over every bank) and a face's four
+// cells are `step` slots apart.
+// ---------------------------------------------------------------------------
+template <int NS>
+constexpr int SLOT = (NS + 4) | 1;
+
+constexpr bool staged(int eos, int recon) { return recon == RECON_MUSCL && eos != EOS_REAL; }
+
+template <int NS>
+struct SlotStencil {
+  const double *s;  // the face's LL cell
+  int step;
+  __device__ __forceinline__ double operator()(int v, int m) const { return s[m * step * SLOT<NS> + v]; }
+};
+
+// one axis's faces in tiles: nf (i) or the log of wi (j, k)
+struct FaceTiles {
+  int axis, shape;
+  Box3 b;
+  FastDiv row, run, plane;  // i: by the row's faces, its cells, the box's rows. j, k: by the tiles along i, along the axis
+};
+
+__host__ inline unsigned face_tile_slots(const FaceTiles &t) {
+  if (t.axis == 0) return (unsigned)(t.shape + 3 * std::min(t.shape, (t.shape - 2) / t.b.e0 + 2));
+  return (1u << t.shape) * ((unsigned)(FLAT >> t.shape) + 3);
+}
+
+__host__ inline int64_t face_tile_count(const FaceTiles &t) {
+  const Box3 &b = t.b;
+  if (t.axis == 0) return ((int64_t)b.e0 * b.e1 * b.e2 + t.shape - 1) / t.shape;
+  const int wi = 1 << t.shape, ta = FLAT / wi;
+  const int64_t ea = t.axis == 1 ? b.e1 : b.e2, eo = t.axis == 1 ? b.e2 : b.e1;
+  return (int64_t)((b.e0 + wi - 1) / wi) * ((ea + ta - 1) / ta) * eo;
+}
+
+// The tile shape of a box's faces. i: 256 faces, fewer where short rows would bring more than 352 slots
+// (36 KB for nine species: four workgroups a CU keep their four waves a SIMD). j, k: the width whose waves
+// and staged cells cost least, a wave of faces taken as eight times its 64 lanes' staging
+__host__ inline FaceTiles face_tiles(int axis, const Box3 &b) {
+  FaceTiles t{axis, 256, b, {}, {}, {}};
+  if (axis == 0) {
+    while (t.shape > 64 && face_tile_slots(t) > 352) t.shape /= 2;
+    t.row = fast_div(b.e0), t.run = fast_div(b.e0 + 3), t.plane = fast_div(b.e1);
+    return t;
+  }
+  const int64_t ea = axis == 1 ? b.e1 : b.e2;
+  int64_t least = 0;
+  for (int s = 4; s <= 6; s++) {
+    const int64_t wi = 1 << s, ta = FLAT / wi, nbi = (b.e0 + wi - 1) / wi, full = ea / ta, rem = ea % ta;
+    const int64_t waves = nbi * (full * (FLAT / 64) + (rem * wi + 63) / 64);
+    const int64_t cost = waves * 64 * 8 + nbi * wi * (ea + 3 * (full + (rem > 0)));
+    if (s == 4 || cost < least) least = cost, t.shape = s;
+  }
+  const unsigned wi = 1u << t.shape, ta = FLAT / wi;
+  t.row = fast_div((b.e0 + wi - 1) / wi), t.run = fast_div((unsigned)(ea + ta - 1) / ta);
+  return t;
+}
+
+// Stages tile t's cells into lds and gives the thread its face: false for a thread with none. Ends in a
+// barrier that every thread of the workgroup passes.
+template <int NS>
+__device__ __forceinline__ bool face_tile(const FaceTiles &ft, unsigned t, const View &Q, const View &st, double *lds,
+                                          int &i, int &j, int &k, SlotStencil<NS> &x) {
+#pragma clang fp contract(off)
+  const Box3 &b = ft.b;
+  const unsigned tid = threadIdx.x, e0 = b.e0, e1 = b.e1;
+  unsigned nslot, slot;
+  bool on;
+  // slot q's cell
+  unsigned col0 = 0, row0 = 0, len0 = 0, ibeg = 0, abeg = 0;
+  int fixed = 0;
+  if (ft.axis == 0) {
+    const unsigned f0 = t * (unsigned)ft.shape, total = e0 * e1 * (unsigned)b.e2;
+    const unsigned n = min((unsigned)ft.shape, total - f0);
+    row0 = ft.row(f0), col0 = f0 - row0 * e0;
+    len0 = min(e0 - col0, n) + 3;
+    nslot = n + 3 * (ft.row(col0 + n - 1) + 1);
+    const unsigned c = col0 + tid, seg = ft.row(c), row = row0 + seg, p = ft.plane(row);
+    on = tid < n;
+    slot = tid + 3 * seg;
+    i = b.s0 + (int)(c - seg * e0), j = b.s1 + (int)(row - p * e1), k = b.s2 + (int)p;
+    x.step = 1;
+  } else {
+    const unsigned lw = ft.shape, wi = 1u << lw, ta = FLAT >> lw;
+    const unsigned ea = ft.axis == 1 ? e1 : (unsigned)b.e2;
+    const unsigned rest = ft.row(t);
+    ibeg = (t - rest * ft.row.d) << lw, fixed = (int)ft.run(rest), abeg = (rest - (unsigned)fixed * ft.run.d) * ta;
+    const unsigned na = min(ta, ea - abeg), ii = ibeg + (tid & (wi - 1)), aa = tid >> lw;
+    on = ii < e0 && aa < na;
+    nslot = (na + 3) << lw;
+    slot = tid;
+    i = b.s0 + (int)ii;
+    j = b.s1 + (ft.axis == 1 ? (int)(abeg + aa) : fixed), k = b.s2 + (ft.axis == 1 ? fixed : (int)(abeg + aa));
+    x.step = (int)wi;
+  }
+  const auto cell = [&](unsigned q) -> int64_t {
+    if (ft.axis == 0) {
+      const bool first = q < len0;
+      const unsigned r = first ? 0 : q - len0, seg = ft.run(r);
+      const unsigned row = first ? row0 : row0 + 1 + seg, p = ft.plane(row);
+      const int ci = first ? (int)(col0 + q) - 2 : (int)(r - seg * (e0 + 3)) - 2;
+      return Q.off(b.s0 + ci, b.s1 + (int)(row - p * e1), b.s2 + (int)p);
+    }
+    // columns past the box repeat its last
+    const int ci = b.s0 + (int)min(ibeg + (q & ((1u << ft.shape) - 1)), e0 - 1), ca = (int)(abeg + (q >> ft.shape)) - 2;
+    return ft.axis == 1 ? Q.off(ci, b.s1 + ca, b.s2 + fixed) : Q.off(ci, b.s1 + fixed, b.s2 + ca);
+  };
+  const auto load = [&](unsigned q, double (&r)[NS + 5]) {
+    uint32_t o = View::bytes(cell(q));
+    r[NS + 4] = st.run(o, 2);
+    r[0] = st.run(o, 0), r[1] = st.run(o, 1);
 #pragma unroll
-  for (int l = 0; l < NS + 4; l++) __builtin_nontemporal_store(Fv[l], &F.at(oF, l));
+    for (int c = 1; c < 4; c++) r[1 + c] = Q.run(o, c);
+#pragma unroll
+    for (int n = 0; n < NS - 1; n++) r[5 + n] = Q.run(o, 5 + n);
+  };
+  const auto put = [&](unsigned q, const double (&r)[NS + 5]) {
+    double *s = lds + q * SLOT<NS>;
+    s[0] = r[0], s[1] = r[1];
+#pragma unroll
+    for (int v = 2; v < NS + 4; v++) s[v] = r[v] * r[NS + 4];
+  };
+  for (unsigned q = tid; q < nslot; q += 2 * FLAT) {
+    double r0[NS + 5], r1[NS + 5];
+    load(q, r0);
+    const bool two = q + FLAT < nslot;
+    if (two) load(q + FLAT, r1);
+    put(q, r0);
+    if (two) put(q + FLAT, r1);
+  }
+  __syncthreads();
+  x.s = lds + slot * SLOT<NS>;
+  return on;
+}
+
+// the flux of face (i, j, k) from its staged stencil
+template <int NS, int EOS, int PRIMARY, int LIM>
+__device__ __forceinline__ void flux_slots(const double *__restrict__ K, const SlotStencil<NS> &x, const View &S, int i,
+                                           int j, int k, double (&Fv)[NS + 4]) {
+  double Sv[3];
+  load_area(S, i, j, k, Sv);
+  FaceState<NS> L, R;
+  muscl_sides<NS, EOS, LIM>(Gas<NS>{K}, x, L, R);
+  flux_function<NS, PRIMARY>(L, R, Sv, Fv);
 }
 
 }  // namespace pga

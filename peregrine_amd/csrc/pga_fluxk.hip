@@ -1,14 +1,12 @@
-// The advective face flux of the per-kernel path: one launch per axis over the
-// faces of a box, one face per thread, lanes along the contiguous i index so the
+// The advective face flux: one launch per axis over the faces of a box (the per-kernel path), or one
+// launch for every face of a block, one face per thread, lanes along the contiguous i index so the
 // stencil reads of every axis are coalesced.
 //
-// The i and j faces take a flat launch (rows of faces back to back, XCD-ordered
-// blocks): the rows a j-face stencil spans are shared with the blocks dispatched
-// beside it on the same XCD, so L2 serves the reuse. A k-face stencil spans four
-// planes, further apart than an XCD's blocks in flight reach: there a workgroup
-// takes a 64 (i) x 4 (k) tile of faces, its four waves four consecutive k-faces,
-// and the seven planes of cells they span are read once into L1 and L2 for all
-// four rather than four times.
+// MUSCL's faces go in tiles whose cells are staged in LDS (face_tile, pga_flux.hpp), but the cubic gas's.
+// Its stencils, and the constant reconstruction's two cells, are read as they are: the i and j faces take
+// a flat launch (rows of faces back to back, XCD-ordered blocks, so the rows a j face shares with its
+// neighbours are read by blocks of the same XCD), and the k faces 64 (i) x 4 (k) tiles, whose four waves
+// share their planes.
 #include "pga_diff.hpp"
 #include "pga_flux.hpp"
 #include "pga_internal.hpp"
@@ -23,18 +21,27 @@ __host__ inline dim3 ktile_grid(const Box3 &b) {
 
 template <int NS, int EOS, int RECON, int PRIMARY, int LIM>
 __global__ __launch_bounds__(256) void k_flux(const double *__restrict__ K, int axis, View Q, View st, View S,
-                                              View F, Box3 b) {
+                                              View F, Box3 b, FaceTiles ft) {
   int i, j, k;
-  if (axis == 2) {
-    const unsigned t = xcd_block(), nbi = (b.e0 + 63) / 64, rest = t / nbi, nkt = (b.e2 + KTILE - 1) / KTILE;
-    i = b.s0 + (int)(t % nbi) * 64 + (threadIdx.x & 63);
-    k = b.s2 + (int)(rest % nkt) * KTILE + (threadIdx.x >> 6);
-    j = b.s1 + (int)(rest / nkt);
-    if (i >= b.s0 + b.e0 || k >= b.s2 + b.e2) return;
-  } else if (!flat_cell_of(b, i, j, k)) {
-    return;
+  if constexpr (staged(EOS, RECON)) {
+    extern __shared__ double lds[];
+    SlotStencil<NS> x;
+    if (!face_tile<NS>(ft, xcd_block(), Q, st, lds, i, j, k, x)) return;
+    double Fv[NS + 4];
+    flux_slots<NS, EOS, PRIMARY, LIM>(K, x, S, i, j, k, Fv);
+    store_flux<NS>(F, i, j, k, Fv);
+  } else {
+    if (axis == 2) {
+      const unsigned t = xcd_block(), nbi = (b.e0 + 63) / 64, rest = t / nbi, nkt = (b.e2 + KTILE - 1) / KTILE;
+      i = b.s0 + (int)(t % nbi) * 64 + (threadIdx.x & 63);
+      k = b.s2 + (int)(rest % nkt) * KTILE + (threadIdx.x >> 6);
+      j = b.s1 + (int)(rest / nkt);
+      if (i >= b.s0 + b.e0 || k >= b.s2 + b.e2) return;
+    } else if (!flat_cell_of(b, i, j, k)) {
+      return;
+    }
+    flux_face<NS, EOS, RECON, PRIMARY, LIM>(K, axis, Q, st, S, F, i, j, k);
   }
-  flux_face<NS, EOS, RECON, PRIMARY, LIM>(K, axis, Q, st, S, F, i, j, k);
 }
 
 // every face of a block in one launch: the i faces' workgroups, then the j faces', then the k faces'
@@ -43,7 +50,7 @@ __global__ __launch_bounds__(256) void k_flux(const double *__restrict__ K, int 
 struct FacesArgs {
   const double *K;
   View Q, st, S0, S1, S2, F0, F1, F2;
-  Box3 b0, b1, b2;
+  FaceTiles t[3];
   unsigned n0, n1;
   double alpha;
   View tr, hsp, gr, xcc, xf0, xf1, xf2;
@@ -52,48 +59,48 @@ struct FacesArgs {
 template <int NS, int EOS, int RECON, int PRIMARY, int LIM, bool VISC>
 __global__ __launch_bounds__(256) void k_faces(FacesArgs a) {
   const unsigned g = xcd_block();
-  int axis, i, j, k;
-  if (g < a.n0) {
-    axis = 0;
-    if (!flat_at(a.b0, g, i, j, k)) return;
-  } else if (g < a.n0 + a.n1) {
-    axis = 1;
-    if (!flat_at(a.b1, g - a.n0, i, j, k)) return;
-  } else {
-    axis = 2;
-    // a column's k tiles one after another: the next tile's workgroup finds three of its seven
-    // planes of cells in L2
-    const Box3 &b = a.b2;
-    const unsigned t = g - a.n0 - a.n1, nbi = (b.e0 + 63) / 64, rest = t / nbi, nkt = (b.e2 + KTILE - 1) / KTILE;
-    i = b.s0 + (int)(t % nbi) * 64 + (threadIdx.x & 63);
-    k = b.s2 + (int)(rest % nkt) * KTILE + (threadIdx.x >> 6);
-    j = b.s1 + (int)(rest / nkt);
-    if (i >= b.s0 + b.e0 || k >= b.s2 + b.e2) return;
-  }
+  const int axis = g < a.n0 ? 0 : g < a.n0 + a.n1 ? 1 : 2;
+  const unsigned t = axis == 0 ? g : axis == 1 ? g - a.n0 : g - a.n0 - a.n1;
   const View &S = axis == 0 ? a.S0 : axis == 1 ? a.S1 : a.S2;
   const View &F = axis == 0 ? a.F0 : axis == 1 ? a.F1 : a.F2;
+  int i, j, k;
   double Fv[NS + 4];
-  flux_at<NS, EOS, RECON, PRIMARY, LIM>(a.K, axis, a.Q, a.st, S, i, j, k, Fv);
+  if constexpr (staged(EOS, RECON)) {
+    extern __shared__ double lds[];
+    SlotStencil<NS> x;
+    if (!face_tile<NS>(a.t[axis], t, a.Q, a.st, lds, i, j, k, x)) return;
+    flux_slots<NS, EOS, PRIMARY, LIM>(a.K, x, S, i, j, k, Fv);
+  } else {
+    const Box3 &b = a.t[axis].b;
+    if (axis < 2) {
+      if (!flat_at(b, t, i, j, k)) return;
+    } else {
+      // a column's k tiles one after another: the next tile's workgroup finds planes of cells in L2
+      const unsigned nbi = (b.e0 + 63) / 64, rest = t / nbi, nkt = (b.e2 + KTILE - 1) / KTILE;
+      i = b.s0 + (int)(t % nbi) * 64 + (threadIdx.x & 63);
+      k = b.s2 + (int)(rest % nkt) * KTILE + (threadIdx.x >> 6);
+      j = b.s1 + (int)(rest / nkt);
+      if (i >= b.s0 + b.e0 || k >= b.s2 + b.e2) return;
+    }
+    flux_at<NS, EOS, RECON, PRIMARY, LIM>(a.K, axis, a.Q, a.st, S, i, j, k, Fv);
+  }
   if constexpr (VISC) {
     const View &xf = axis == 0 ? a.xf0 : axis == 1 ? a.xf1 : a.xf2;
     diff_face<NS>(a.Q, a.st, a.tr, a.hsp, a.gr, a.xcc, xf, S, a.alpha, axis, i, j, k, Fv);
   }
-  // the face array streams past the caches: the stencil's Q and state keep L2 (5% on the 128^3 step's
-  // faces); the stage reads the array back from HBM either way
-  const int64_t oF = F.off(i, j, k);
-#pragma unroll
-  for (int l = 0; l < NS + 4; l++) __builtin_nontemporal_store(Fv[l], &F.at(oF, l));
+  store_flux<NS>(F, i, j, k, Fv);
 }
 
 template <int NS, int EOS>
-static void launch_faces(const pga_case *c, const FacesArgs &a, bool visc, dim3 grid, hipStream_t s) {
+static void launch_faces(const pga_case *c, const FacesArgs &a, bool visc, dim3 grid, unsigned slots, hipStream_t s) {
   const int lim = c->desc.limiter, recon = c->desc.recon, prim = c->desc.primary;
+  const size_t lds = sizeof(double) * slots * SLOT<NS>;
 #define L(RECON, PRIM, LIM)                                                                                    \
   if (recon == RECON && prim == PRIM && (RECON == RECON_CONSTANT || lim == LIM)) {                            \
     if (visc)                                                                                                  \
-      hipLaunchKernelGGL((k_faces<NS, EOS, RECON, PRIM, LIM, true>), grid, dim3(FLAT), 0, s, a);               \
+      hipLaunchKernelGGL((k_faces<NS, EOS, RECON, PRIM, LIM, true>), grid, dim3(FLAT), lds, s, a);             \
     else                                                                                                       \
-      hipLaunchKernelGGL((k_faces<NS, EOS, RECON, PRIM, LIM, false>), grid, dim3(FLAT), 0, s, a);              \
+      hipLaunchKernelGGL((k_faces<NS, EOS, RECON, PRIM, LIM, false>), grid, dim3(FLAT), lds, s, a);            \
   }
   L(RECON_CONSTANT, FLUX_KEPAEC, LIM_NONE)
   L(RECON_CONSTANT, FLUX_HLLC, LIM_NONE)
@@ -111,12 +118,14 @@ template <int NS, int EOS>
 static void launch_flux(const pga_case *c, int axis, pga_view Q, pga_view st, pga_view S, pga_view F, Box3 b,
                         hipStream_t s) {
   const int lim = c->desc.limiter, recon = c->desc.recon, prim = c->desc.primary;
+  const FaceTiles ft = face_tiles(axis, b);
+  const bool tiles = staged(EOS, recon);
+  const dim3 grid = tiles ? dim3((unsigned)face_tile_count(ft)) : axis == 2 ? ktile_grid(b) : flat_grid(b);
+  const size_t lds = tiles ? sizeof(double) * face_tile_slots(ft) * SLOT<NS> : 0;
 #define L(RECON, PRIM, LIM)                                                                                    \
   if (recon == RECON && prim == PRIM && (RECON == RECON_CONSTANT || lim == LIM))                              \
-    flat_slabs(b, [&](const Box3 &sb) {                                                                        \
-      hipLaunchKernelGGL((k_flux<NS, EOS, RECON, PRIM, LIM>), axis == 2 ? ktile_grid(sb) : flat_grid(sb),       \
-                         dim3(FLAT), 0, s, c->K, axis, view(Q), view(st), view(S), view(F), sb);                \
-    });
+    hipLaunchKernelGGL((k_flux<NS, EOS, RECON, PRIM, LIM>), grid, dim3(FLAT), lds, s, c->K, axis, view(Q),      \
+                       view(st), view(S), view(F), b, ft);
   L(RECON_CONSTANT, FLUX_KEPAEC, LIM_NONE)
   L(RECON_CONSTANT, FLUX_HLLC, LIM_NONE)
   L(RECON_CONSTANT, FLUX_RUSANOV, LIM_NONE)
@@ -206,10 +215,19 @@ extern "C" int32_t pga_faces(const pga_case *c, pga_view Q, pga_view state, cons
   a.Q = view(Q), a.st = view(state);
   a.S0 = view(S[0]), a.S1 = view(S[1]), a.S2 = view(S[2]);
   a.F0 = view(F[0]), a.F1 = view(F[1]), a.F2 = view(F[2]);
-  a.b0 = box3(boxes[0]), a.b1 = box3(boxes[1]), a.b2 = box3(boxes[2]);
-  a.n0 = empty(boxes[0]) ? 0 : flat_grid(a.b0).x;
-  a.n1 = empty(boxes[1]) ? 0 : flat_grid(a.b1).x;
-  const unsigned n2 = empty(boxes[2]) ? 0 : ktile_grid(a.b2).x;
+  unsigned n[3] = {0, 0, 0}, slots = 0;
+  for (int axis = 0; axis < 3; axis++) {
+    if (empty(boxes[axis])) continue;
+    a.t[axis] = face_tiles(axis, box3(boxes[axis]));
+    if (staged(d.eos, d.recon)) {
+      n[axis] = (unsigned)face_tile_count(a.t[axis]);
+      slots = std::max(slots, face_tile_slots(a.t[axis]));
+    } else {
+      n[axis] = axis == 2 ? ktile_grid(a.t[axis].b).x : flat_grid(a.t[axis].b).x;
+    }
+  }
+  a.n0 = n[0], a.n1 = n[1];
+  const unsigned n2 = n[2];
   if (viscous) {
     a.alpha = alpha;
     a.tr = view(trstate), a.hsp = view(hsp), a.gr = view(grads), a.xcc = view(xcc);
@@ -217,7 +235,7 @@ extern "C" int32_t pga_faces(const pga_case *c, pga_view Q, pga_view state, cons
   }
   const unsigned total = a.n0 + a.n1 + n2;
   if (!total) return PGA_OK;
-  const bool done = dispatch_eos(d, [&]<int N, int E>() { launch_faces<N, E>(c, a, viscous != 0, dim3(total), stream_of(stream)); });
+  const bool done = dispatch_eos(d, [&]<int N, int E>() { launch_faces<N, E>(c, a, viscous != 0, dim3(total), slots, stream_of(stream)); });
   if (!done) {
     set_error("pga_faces: no kernel for %d species with eos %d", d.ns, d.eos);
     return PGA_EUNSUP;
