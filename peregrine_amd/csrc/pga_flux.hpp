@@ -242,20 +242,26 @@ __device__ __forceinline__ void store_flux(const View &F, int i, int j, int k, c
   for (int l = 0; l < NS + 4; l++) __builtin_nontemporal_store(Fv[l], &F.run(b, l));
 }
 
-// the face (i, j, k) of `axis` (between cells k - 1 and k along it): its sides, its flux into Fv
+// the face (i, j, k) of `axis` (between cells k - 1 and k along it): its sides, its area into Sv and its
+// flux into Fv
 template <int NS, int EOS, int RECON, int PRIMARY, int LIM>
 __device__ __forceinline__ void flux_at(const double *__restrict__ K, int axis, const View &Q, const View &st,
-                                        const View &S, int i, int j, int k, double (&Fv)[NS + 4]) {
+                                        const View &S, int i, int j, int k, double (&Sv)[3], double (&Fv)[NS + 4]) {
   const Gas<NS> g{K};
   const int64_t o = Q.off(i, j, k);
   const int64_t d = axis == 0 ? 1 : axis == 1 ? Q.sj : Q.sk;
   FaceState<NS> L, R;
-  if constexpr (RECON == RECON_CONSTANT)
+  // the constant reconstruction's face waits on memory once, its area among the cells' values and cached: a
+  // small block's areas stay in L2 from stage to stage
+  if constexpr (RECON == RECON_CONSTANT) {
+    uint32_t b = View::bytes(S.off(i, j, k));
+#pragma unroll
+    for (int m = 0; m < 3; m++) Sv[m] = S.run(b, m);
     constant_sides<NS>(Q, st, o, d, L, R);
-  else
+  } else {
     muscl_sides<NS, EOS, LIM>(g, ArrayStencil<NS>(Q, st, o, d), L, R);
-  double Sv[3];
-  load_area(S, i, j, k, Sv);
+    load_area(S, i, j, k, Sv);
+  }
   flux_function<NS, PRIMARY>(L, R, Sv, Fv);
 }
 
@@ -263,8 +269,8 @@ __device__ __forceinline__ void flux_at(const double *__restrict__ K, int axis, 
 template <int NS, int EOS, int RECON, int PRIMARY, int LIM>
 __device__ __forceinline__ void flux_face(const double *__restrict__ K, int axis, const View &Q, const View &st,
                                           const View &S, const View &F, int i, int j, int k) {
-  double Fv[NS + 4];
-  flux_at<NS, EOS, RECON, PRIMARY, LIM>(K, axis, Q, st, S, i, j, k, Fv);
+  double Sv[3], Fv[NS + 4];
+  flux_at<NS, EOS, RECON, PRIMARY, LIM>(K, axis, Q, st, S, i, j, k, Sv, Fv);
   store_flux<NS>(F, i, j, k, Fv);
 }
 
@@ -417,11 +423,10 @@ __device__ __forceinline__ bool face_tile(const FaceTiles &ft, unsigned t, const
   return on;
 }
 
-// the flux of face (i, j, k) from its staged stencil
+// the area Sv and flux Fv of face (i, j, k) from its staged stencil
 template <int NS, int EOS, int PRIMARY, int LIM>
 __device__ __forceinline__ void flux_slots(const double *__restrict__ K, const SlotStencil<NS> &x, const View &S, int i,
-                                           int j, int k, double (&Fv)[NS + 4]) {
-  double Sv[3];
+                                           int j, int k, double (&Sv)[3], double (&Fv)[NS + 4]) {
   load_area(S, i, j, k, Sv);
   FaceState<NS> L, R;
   muscl_sides<NS, EOS, LIM>(Gas<NS>{K}, x, L, R);

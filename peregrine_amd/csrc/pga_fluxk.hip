@@ -27,8 +27,8 @@ __global__ __launch_bounds__(256) void k_flux(const double *__restrict__ K, int 
     extern __shared__ double lds[];
     SlotStencil<NS> x;
     if (!face_tile<NS>(ft, xcd_block(), Q, st, lds, i, j, k, x)) return;
-    double Fv[NS + 4];
-    flux_slots<NS, EOS, PRIMARY, LIM>(K, x, S, i, j, k, Fv);
+    double Sv[3], Fv[NS + 4];
+    flux_slots<NS, EOS, PRIMARY, LIM>(K, x, S, i, j, k, Sv, Fv);
     store_flux<NS>(F, i, j, k, Fv);
   } else {
     if (axis == 2) {
@@ -63,30 +63,40 @@ __global__ __launch_bounds__(256) void k_faces(FacesArgs a) {
   const unsigned t = axis == 0 ? g : axis == 1 ? g - a.n0 : g - a.n0 - a.n1;
   const View &S = axis == 0 ? a.S0 : axis == 1 ? a.S1 : a.S2;
   const View &F = axis == 0 ? a.F0 : axis == 1 ? a.F1 : a.F2;
+  const View &xf = axis == 0 ? a.xf0 : axis == 1 ? a.xf1 : a.xf2;
   int i, j, k;
-  double Fv[NS + 4];
+  double Sv[3], Fv[NS + 4];
+  DiffRows rows;
+  // a face of few values reads everything ahead of both fluxes, one wait in all; MUSCL's sides and their
+  // EOS want the registers first
+  constexpr bool ahead = VISC && RECON == RECON_CONSTANT && NS <= 3;
   if constexpr (staged(EOS, RECON)) {
     extern __shared__ double lds[];
     SlotStencil<NS> x;
     if (!face_tile<NS>(a.t[axis], t, a.Q, a.st, lds, i, j, k, x)) return;
-    flux_slots<NS, EOS, PRIMARY, LIM>(a.K, x, S, i, j, k, Fv);
+    flux_slots<NS, EOS, PRIMARY, LIM>(a.K, x, S, i, j, k, Sv, Fv);
   } else {
-    const Box3 &b = a.t[axis].b;
-    if (axis < 2) {
-      if (!flat_at(b, t, i, j, k)) return;
+    // each axis's box named outright: indexed by the axis, its scalar loads would wait for the axis first
+    if (axis == 0) {
+      if (!flat_at(a.t[0].b, t, i, j, k)) return;
+    } else if (axis == 1) {
+      if (!flat_at(a.t[1].b, t, i, j, k)) return;
     } else {
       // a column's k tiles one after another: the next tile's workgroup finds planes of cells in L2
+      const Box3 &b = a.t[2].b;
       const unsigned nbi = (b.e0 + 63) / 64, rest = t / nbi, nkt = (b.e2 + KTILE - 1) / KTILE;
       i = b.s0 + (int)(t % nbi) * 64 + (threadIdx.x & 63);
       k = b.s2 + (int)(rest % nkt) * KTILE + (threadIdx.x >> 6);
       j = b.s1 + (int)(rest / nkt);
       if (i >= b.s0 + b.e0 || k >= b.s2 + b.e2) return;
     }
-    flux_at<NS, EOS, RECON, PRIMARY, LIM>(a.K, axis, a.Q, a.st, S, i, j, k, Fv);
+    if constexpr (ahead) diff_load<NS>(a.tr, a.hsp, a.gr, a.xcc, xf, diff_at(a.Q, xf, axis, i, j, k), rows);
+    flux_at<NS, EOS, RECON, PRIMARY, LIM>(a.K, axis, a.Q, a.st, S, i, j, k, Sv, Fv);
   }
   if constexpr (VISC) {
-    const View &xf = axis == 0 ? a.xf0 : axis == 1 ? a.xf1 : a.xf2;
-    diff_face<NS>(a.Q, a.st, a.tr, a.hsp, a.gr, a.xcc, xf, S, a.alpha, axis, i, j, k, Fv);
+    const DiffAt at = diff_at(a.Q, xf, axis, i, j, k);
+    if constexpr (!ahead) diff_load<NS>(a.tr, a.hsp, a.gr, a.xcc, xf, at, rows);
+    diff_face<NS>(a.Q, a.st, a.tr, a.hsp, a.gr, rows, at, Sv, a.alpha, Fv);
   }
   store_flux<NS>(F, i, j, k, Fv);
 }

@@ -190,8 +190,8 @@ __device__ __forceinline__ void march_cells(const StageArgs &a, const View &kS, 
   const double dt = *a.dt;
   int lo = 0;
   {
-    double Fv[NE];
-    flux_at<NS, EOS, RECON, PRIMARY, LIM>(a.K, 2, a.Qin, a.stin, kS, i, j, kbeg, Fv);
+    double Sv[3], Fv[NE];
+    flux_at<NS, EOS, RECON, PRIMARY, LIM>(a.K, 2, a.Qin, a.stin, kS, i, j, kbeg, Sv, Fv);
 #pragma unroll
     for (int l = 0; l < NE; l++) lds[(lo * NE + l) * WT + tid] = Fv[l];
   }
@@ -199,8 +199,8 @@ __device__ __forceinline__ void march_cells(const StageArgs &a, const View &kS, 
   for (int k = kbeg; k < kend; k++) {
     const int hi = lo ^ 1;
     {
-      double Fv[NE];
-      flux_at<NS, EOS, RECON, PRIMARY, LIM>(opaque(a.K), 2, a.Qin, a.stin, kS, i, j, k + 1, Fv);
+      double Sv[3], Fv[NE];
+      flux_at<NS, EOS, RECON, PRIMARY, LIM>(opaque(a.K), 2, a.Qin, a.stin, kS, i, j, k + 1, Sv, Fv);
 #pragma unroll
       for (int l = 0; l < NE; l++) lds[(hi * NE + l) * WT + tid] = Fv[l];
     }

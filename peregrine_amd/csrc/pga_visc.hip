@@ -297,7 +297,12 @@ __global__ __launch_bounds__(256) void k_diffflux(DiffArgs a) {
 #pragma unroll
   for (int l = 1; l < NS + 4; l++) Fv[l] = a.F.at(off_, l);
   Fv[0] = 0.0;
-  diff_face<NS>(a.Q, a.st, a.tr, a.hsp, a.gr, a.xcc, a.xf, a.S, a.alpha, AXIS, i, j, k, Fv);
+  const int64_t ofa = a.S.off(i, j, k);
+  const double Sv[3] = {a.S.at(ofa, 0), a.S.at(ofa, 1), a.S.at(ofa, 2)};
+  const DiffAt at = diff_at(a.Q, a.xf, AXIS, i, j, k);
+  DiffRows rows;
+  diff_load<NS>(a.tr, a.hsp, a.gr, a.xcc, a.xf, at, rows);
+  diff_face<NS>(a.Q, a.st, a.tr, a.hsp, a.gr, rows, at, Sv, a.alpha, Fv);
 #pragma unroll
   for (int l = 1; l < NS + 4; l++) a.F.at(off_, l) = Fv[l];
 }
