@@ -168,37 +168,30 @@ __global__ __launch_bounds__(FLAT) void kb_stage(BArgs a, BStage s) {
 }
 
 // implicit chemistry over every block's cells into their rates: a cell's place in the work arrays is
-// its workgroup's flat number times 256 plus its lane, the same in both launches
+// its 256-cell tile's flat number times 256 plus its number in the tile, the same in every launch
 template <class M>
-__global__ __launch_bounds__(FLAT) void kb_itc(BArgs a, ImArgs im) {
-  const int64_t g = xcd_block();
-  const int n = bfind(a.prefix, a.nblocks, g);
-  const BBlock &B = a.blocks[n];
-  int i, j, k;
-  if (!flat_at(B.b, g - a.prefix[n], i, j, k)) return;
-  ijac_tcache<M>(im, B.Q[a.q], B.st, i, j, k, g * FLAT + threadIdx.x);
-}
-
-template <class M>
-__global__ __launch_bounds__(FLAT) void kb_ibase(BArgs a, ImArgs im) {
-  const int64_t g = xcd_block();
-  const int n = bfind(a.prefix, a.nblocks, g);
-  const BBlock &B = a.blocks[n];
-  int i, j, k;
-  if (!flat_at(B.b, g - a.prefix[n], i, j, k)) return;
-  ijac_base<M>(im, B.Q[a.q], i, j, k, g * FLAT + threadIdx.x);
-}
-
-// a tile's slices (the ns + 1 columns and f(y)) in workgroups numbered one after another, as k_icol
-template <class M>
-__global__ __launch_bounds__(FLAT) void kb_icol(BArgs a, ImArgs im) {
-  constexpr int64_t S = M::NS + 2;
+__global__ __launch_bounds__(M::GROUPS *IM_CELLS) void kb_icol(BArgs a, ImArgs im) {
+  extern __shared__ double lds[];
+  constexpr int64_t S = FLAT / IM_CELLS;
   const int64_t gs = xcd_block(), g = gs / S;
   const int n = bfind(a.prefix, a.nblocks, g);
   const BBlock &B = a.blocks[n];
+  const unsigned first = (unsigned)(g - a.prefix[n]) * FLAT, cells = (unsigned)B.b.e0 * B.b.e1 * B.b.e2;
+  const unsigned c = min(first + (unsigned)(gs - g * S) * IM_CELLS + threadIdx.x % IM_CELLS, cells - 1);
+  int i, j, k;
+  cell_at(B.b, c, i, j, k);
+  ijac_columns<M>(im, B.Q[a.q], B.st, lds, i, j, k, g * FLAT + (c - first));
+}
+
+// a tile's two slices in workgroups numbered one after another, as k_iwhole
+template <class M>
+__global__ __launch_bounds__(FLAT) void kb_iwhole(BArgs a, ImArgs im) {
+  const int64_t gs = xcd_block(), g = gs / 2;
+  const int n = bfind(a.prefix, a.nblocks, g);
+  const BBlock &B = a.blocks[n];
   int i, j, k;
   if (!flat_at(B.b, g - a.prefix[n], i, j, k)) return;
-  ijac_column<M>(im, B.Q[a.q], i, j, k, g * FLAT + threadIdx.x, (int)(gs - g * S));
+  ijac_whole<M>(im, B.Q[a.q], i, j, k, g * FLAT + threadIdx.x, (int)(gs % 2));
 }
 
 // the places of a tile's overhang (no cell): the identity and a zero right-hand side, once a call,
@@ -535,9 +528,8 @@ static int64_t batch_cells(const pga_batch *h) { return h->total[BK_CELLS] * FLA
 extern "C" int64_t pga_batch_implicit_worksize(const pga_batch *h) {
   if (!h || h->c->desc.ns + 1 > IM_N) return -1;
   const int64_t cells = batch_cells(h), groups = (cells + IM_G - 1) / IM_G, nv = h->c->desc.ns + 1;
-  const int64_t nt = im_cache_doubles(h->c->desc);
-  if (nt < 0) return -1;
-  return groups * nv * nv * IM_G + (3 * nv + nt) * cells;
+  if (h->c->desc.mechanism < 0) return -1;
+  return groups * nv * nv * IM_G + 3 * nv * cells;
 }
 
 extern "C" int32_t pga_batch_implicit(const pga_batch *h, const pga_implicit_opts *o, int32_t q, int32_t *sweeps,
@@ -565,7 +557,6 @@ extern "C" int32_t pga_batch_implicit(const pga_batch *h, const pga_implicit_opt
   im.begin_dQ = 0;
   im.A = work;
   im.y = im.A + groups * nv * nv * IM_G;
-  im.tc = im.y + 3 * nv * cells;
   im.ncell = cells, im.sweeps = sweeps, im.dt = dt;
   im.parts = o->parts, im.maxsweeps = o->max_sweeps, im.tol = o->tolerance;
   const BArgs a = bargs(h, q, q, 0, h->prefix[BK_CELLS]);
@@ -578,9 +569,9 @@ extern "C" int32_t pga_batch_implicit(const pga_batch *h, const pga_implicit_opt
     hipLaunchKernelGGL((kb_ivoid<NV>), grid, dim3(FLAT), 0, s, a, im);                           \
     for (int part = 0; part < o->parts; part++) {                                                \
       im.first = part == 0, im.last = part == o->parts - 1;                                      \
-      hipLaunchKernelGGL((kb_itc<Mech_##NAME>), grid, dim3(FLAT), 0, s, a, im);                 \
-      hipLaunchKernelGGL((kb_ibase<Mech_##NAME>), grid, dim3(FLAT), 0, s, a, im);               \
-      hipLaunchKernelGGL((kb_icol<Mech_##NAME>), dim3(grid.x * (NV + 1)), dim3(FLAT), 0, s, a, im); \
+      hipLaunchKernelGGL((kb_icol<Mech_##NAME>), dim3(grid.x * (FLAT / IM_CELLS)),               \
+                         dim3(Mech_##NAME::GROUPS * IM_CELLS), im_cols_lds<Mech_##NAME>, s, a, im); \
+      hipLaunchKernelGGL((kb_iwhole<Mech_##NAME>), dim3(grid.x * 2), dim3(FLAT), 0, s, a, im);   \
       hipLaunchKernelGGL((k_lusolve<NB, NV>), dim3((unsigned)((groups + 3) / 4)), dim3(256), 0, s, im); \
     }                                                                                            \
     hipLaunchKernelGGL((kb_iend<Mech_##NAME>), grid, dim3(FLAT), 0, s, a, im);                  \

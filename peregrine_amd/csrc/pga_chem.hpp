@@ -10,8 +10,8 @@ namespace pga {
 // g/(Ru T) of species n: its Gibbs polynomial in ln T plus h298/T (eos/kernels/species.mako:16-21),
 // Horner steps as explicit fused multiply-adds (the oracle evaluates the same sequence): the
 // polynomial's terms cancel by six orders, so the rounding sequence is fixed, not left to the compiler
-template <int NS>
-__device__ __forceinline__ double gibbs_rt(const Gas<NS> &g, int n, double logT, double Tinv) {
+template <int NS, class P>
+__device__ __forceinline__ double gibbs_rt(const GasOf<NS, P> &g, int n, double logT, double Tinv) {
 #pragma clang fp contract(off)
   double gr = 0.0;
 #pragma unroll
@@ -20,8 +20,8 @@ __device__ __forceinline__ double gibbs_rt(const Gas<NS> &g, int n, double logT,
 }
 
 // cp/R and the internal energy of species n at T (eos/kernels/species.mako:3-27), u = ln T
-template <int NS>
-__device__ __forceinline__ double cpR_species(const Gas<NS> &g, int n, double u) {
+template <int NS, class P>
+__device__ __forceinline__ double cpR_species(const GasOf<NS, P> &g, int n, double u) {
 #pragma clang fp contract(off)
   double cpR = 0.0;
 #pragma unroll
@@ -29,8 +29,8 @@ __device__ __forceinline__ double cpR_species(const Gas<NS> &g, int n, double u)
   return cpR;
 }
 
-template <int NS>
-__device__ __forceinline__ double e_species(const Gas<NS> &g, int n, double T, double u, double Tinv) {
+template <int NS, class P>
+__device__ __forceinline__ double e_species(const GasOf<NS, P> &g, int n, double T, double u, double Tinv) {
 #pragma clang fp contract(off)
   double hRT = 0.0;
 #pragma unroll

@@ -80,10 +80,10 @@ __host__ __device__ constexpr Offsets offsets(int ns) {
 
 // the species constants of a case with NS species, read at compile-time offsets from a
 // wave-uniform pointer: the compiler turns each read into a scalar load
-template <int NS>
-struct Gas {
+template <int NS, class P>
+struct GasOf {
   static constexpr Offsets O = offsets(NS);
-  const double *__restrict__ K;
+  P K;
   __device__ __forceinline__ double MW(int n) const { return K[O.MW + n]; }
   __device__ __forceinline__ double MWinv(int n) const { return K[O.MWinv + n]; }
   __device__ __forceinline__ double Rsp(int n) const { return K[O.Rsp + n]; }
@@ -125,6 +125,14 @@ struct Gas {
   __device__ __forceinline__ double bathof(int n, int k) const { return K[O.bathof + n * NS + k]; }
   __device__ __forceinline__ double diffmeta(int i) const { return K[O.diffmeta + i]; }
 };
+
+template <int NS>
+using Gas = GasOf<NS, const double *__restrict__>;
+
+// a constant table in the constant address space: its reads are scalar loads wherever they stand, where
+// through a plain pointer they are vector loads, a register pair each, behind a store of another branch
+using Constants = const __attribute__((address_space(4))) double *;
+__device__ __forceinline__ Constants constants(const double *p) { return (Constants)(uintptr_t)p; }
 
 // ---------------------------------------------------------------------------
 // views and launch shapes
@@ -221,6 +229,15 @@ __host__ inline void flat_slabs(const Box3 &b, F &&launch) {
 __device__ __forceinline__ unsigned xcd_block() {
   const unsigned nb = gridDim.x, bid = blockIdx.x, x = bid % NXCD, q = nb / NXCD, r = nb % NXCD;
   return x * q + (x < r ? x : r) + bid / NXCD;
+}
+
+// the c-th cell of box b, i fastest; false past the box
+__device__ __forceinline__ bool cell_at(const Box3 &b, unsigned c, int &i, int &j, int &k) {
+  const unsigned row = c / (unsigned)b.e0;
+  i = b.s0 + (int)(c - row * (unsigned)b.e0);
+  j = b.s1 + (int)(row % (unsigned)b.e1);
+  k = b.s2 + (int)(row / (unsigned)b.e1);
+  return row < (unsigned)b.e1 * (unsigned)b.e2;
 }
 
 __device__ __forceinline__ bool flat_cell_of(const Box3 &b, int &i, int &j, int &k) {

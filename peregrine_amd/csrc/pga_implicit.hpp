@@ -181,7 +181,6 @@ struct ImArgs {
   int begin_dQ, first, last;
   double *A;     // the FP64 matrices, group-major with nv^2 entries
   double *y;     // [ns + 1][ncell] three times: the part's start (then its end), f at its FP32 rounding, f at it
-  double *tc;    // [im_cache_n][ncell]: the cache of f at the FP32 rounding's T
   int64_t ncell;
   int32_t *sweeps;
   const double *dt;
@@ -238,58 +237,6 @@ struct ImCache {
 
 template <class M>
 constexpr int im_cache_n = sizeof(ImCache<M>) / sizeof(double);
-
-// the cache of f at T into tc[entry * nc] in ImCache's order, each value stored as it is made (C, K and
-// tc in one restrict scope, so the constants keep their scalar loads and nothing waits in a register)
-template <class M>
-__device__ __forceinline__ void im_cache_write(const double *__restrict__ K, const double *__restrict__ C, double T,
-                                               double *__restrict__ tc, int64_t nc) {
-#pragma clang fp contract(off)
-  constexpr int NS = M::NS, NT = sizeof(typename M::TCache) / sizeof(double);
-  const Gas<NS> g{K};
-  M::tstate(g, C, T, tc, nc);
-  const double logT = tlog(T), Tinv = 1.0 / T;
-#pragma unroll
-  for (int n = 0; n < NS; n++) {
-    const double cpR = cpR_species(g, n, logT);
-    tc[(NT + n) * nc] = (cpR - 1.0) * g.Rsp(n);
-    tc[(NT + NS + n) * nc] = e_species(g, n, T, logT, Tinv);
-  }
-}
-
-// rhs0d at a composition whose T is the cache's
-template <class M>
-__device__ __forceinline__ void rhs0d_cached(const Gas<M::NS> &g, const double *__restrict__ C, double rho,
-                                             double rhoinv, const double (&y)[M::NS + 1], const ImCache<M> &c,
-                                             double (&f)[M::NS + 1]) {
-#pragma clang fp contract(off)
-  constexpr int NS = M::NS;
-  double Y[NS], rate[NS], D[NS];
-#pragma unroll
-  for (int n = 0; n < NS; n++) Y[n] = y[n];
-  typename M::Rates s;
-  M::cstate(g, C, rho, Y, c.t, s);
-  M::template fold_cached<false>(C, s, c.t, rate, D);
-  double cv = 0.0, dTdt = 0.0;
-#pragma unroll
-  for (int n = 0; n < NS; n++) {
-    cv += c.ea[n] * Y[n];
-    dTdt -= c.ee[n] * rate[n];
-  }
-  const double cvrhoinv = 1.0 / (cv * rho);
-#pragma unroll
-  for (int n = 0; n < NS; n++) f[n] = rate[n] * rhoinv;
-  f[NS] = dTdt * cvrhoinv;
-}
-
-// the cache of work place `code` from the work array's [entry][ncell] region
-template <class M>
-__device__ __forceinline__ void im_cache_load(const double *__restrict__ tc, int64_t nc, int64_t code, ImCache<M> &c) {
-  double v[im_cache_n<M>];
-#pragma unroll
-  for (int e = 0; e < im_cache_n<M>; e++) v[e] = tc[e * nc + code];
-  __builtin_memcpy(&c, v, sizeof(v));
-}
 
 __device__ __forceinline__ int64_t im_code(const Box3 &b, int i, int j, int k) {
   return (i - b.s0) + (int64_t)b.e0 * ((j - b.s1) + (int64_t)b.e1 * (k - b.s2));
@@ -352,98 +299,190 @@ __device__ __forceinline__ int refine(const float *__restrict__ W, const double 
   return done ? s : maxsweeps + 1;
 }
 
-// A = I - h J at the part's start, J by forward differences, in three launches: the cache (a lane per
-// cell) stores y and what f shares over the compositions of y^'s T (y^: y rounded to FP32); the base
-// f(y^); the columns (a lane per cell and unknown) each one column of A, a species column from the
-// cache, the T column by two whole evaluations, and one more slice f(y) itself, the solve's
-// right-hand side. J is taken at y^: a
-// last-bit change of y (the oracle's FP64 solve against the device's refined one, a part's start
-// after another part) then leaves the matrix as it was, where the differences' own rounding would
-// move it by 1e-12 of itself and a stiff part's result by more; the linearly implicit Euler step is
-// first order with the matrix of any nearby state. A lane makes one evaluation of the rates, so the
-// lanes hold the registers of one evaluation and the chip's waves are as many as for the rates alone.
+// A = I - h J at the part's start, J by forward differences, in two launches: the species columns, with y
+// and f(y^) (y^: y rounded to FP32), and then the T column and f(y), the solve's right-hand side, a whole
+// evaluation each. J is taken at y^: a last-bit change of y (the oracle's FP64 solve against the device's
+// refined one, a part's start after another part) then leaves the matrix as it was, where the differences'
+// own rounding would move it by 1e-12 of itself and a stiff part's result by more; the linearly implicit
+// Euler step is first order with the matrix of any nearby state.
+//
+// The species columns: 64 cells a workgroup, a wave a group of M::COLS species. The waves make the cache of
+// y^'s T between them into LDS (a share each, M::tstate_part), then each takes f at y^ and at its group's
+// columns from it, evaluating a reaction again only for the columns whose species it reads
+// (M::fold_columns; each column's sums its own, in order). A lane a column, with the cache in HBM, read its
+// 68 values for every column and was bound by that; three columns a lane reading it from L2 waited on each
+// value in turn (280 us against 191 for 64^3 cells), and from LDS, where the cache never leaves the chip, the
+// two launches take 97 + 69 us for the 64^3 cells in place of 260, at three waves a SIMD. The 64^3 step went
+// from 1.45 to 1.16 ms, that of 16 boxes of 3.0 million cells in all from 16.9 to 13.0 ms.
 
-// the part's start: the first part takes y from Q and the state, a later one the y the last part left
-// (selected rather than branched, one copy of the code); y and the cache of f at y^'s T into the work
-// array, every store after the constants' loads (which then go through the scalar cache)
+constexpr int IM_CELLS = 64;  // cells of a workgroup of the species columns
+
 template <class M>
-__device__ __forceinline__ void ijac_tcache(const ImArgs &a, const View &Q, const View &st, int i, int j, int k,
-                                            int64_t code) {
-#pragma clang fp contract(off)
-  constexpr int NS = M::NS, NV = NS + 1;
-  const int64_t nc = a.ncell;
-  const int64_t o = Q.off(i, j, k);
-  const double rhoinv = 1.0 / Q.at(o, 0);
-  double *y = a.y + code;
-  double y0[NV], Y[NS];
+constexpr size_t im_cols_lds = sizeof(double) * im_cache_n<M> * IM_CELLS;
+
+// the y of a cell at the part's start: the first part's from Q and the state, a later one's as the last part
+// left it (selected rather than branched, one copy of the code)
+template <class M>
+__device__ __forceinline__ void im_y0(const ImArgs &a, const View &Q, const View &st, int64_t o, int64_t ost,
+                                      double rhoinv, int64_t code, double (&y0)[M::NS + 1]) {
+  constexpr int NS = M::NS;
+  double Y[NS];
   massfrac<NS>(Q, o, rhoinv, Y);
 #pragma unroll
-  for (int n = 0; n < NS; n++) y0[n] = a.first ? Y[n] : y[n * nc];
-  y0[NS] = a.first ? st.at(st.off(i, j, k), 1) : y[NS * nc];
-  im_cache_write<M>(a.K, a.C, (double)(float)y0[NS], a.tc + code, nc);
-#pragma unroll
-  for (int r = 0; r < NV; r++) y[r * nc] = y0[r];
+  for (int n = 0; n < NS; n++) y0[n] = a.first ? Y[n] : a.y[n * a.ncell + code];
+  y0[NS] = a.first ? st.at(ost, 1) : a.y[NS * a.ncell + code];
 }
 
-// the base: f at y rounded to FP32 (y^), from the cache, into the work array
+// a wave's view of the constants and of its lane's place in the cache, as values the compiler cannot match
+// with another group's: it would read what the groups share ahead of the branch that tells them apart, and
+// hold it in registers 
+struct ImGroup {
+  Constants K, C;
+  double *lds;
+  unsigned lane;
+  __device__ __forceinline__ ImGroup(const ImArgs &a, double *l) : K(constants(a.K)), C(constants(a.C)), lds(l) {
+    lane = threadIdx.x % IM_CELLS;
+    asm volatile("" : "+s"(K), "+s"(C), "+v"(lane));
+  }
+  // entry e of the lane's cell
+  __device__ __forceinline__ double &operator()(int e) const { return lds[e * IM_CELLS + lane]; }
+};
+
+// ends a group's branch: without it the stores that end every branch are made one store where they join,
+// with every value waiting in registers
+__device__ __forceinline__ void im_branch_end() { asm volatile(""); }
+
+// group G's share of a cell's cache at T
+template <class M, int G>
+__device__ __forceinline__ void ijac_part(const ImArgs &a, double T, double *lds) {
+#pragma clang fp contract(off)
+  constexpr int NS = M::NS, NT = sizeof(typename M::TCache) / sizeof(double);
+  const ImGroup X(a, lds);
+  const GasOf<NS, Constants> g{X.K};
+  const auto put = [&](int e, double v) { X(e) = v; };
+  M::template tstate_part<G>(g, X.C, T, put);
+  const double logT = tlog(T), Tinv = 1.0 / T;
+#pragma unroll
+  for (int n = G; n < NS; n += M::GROUPS) {
+    const double cpR = cpR_species(g, n, logT);
+    put(NT + n, (cpR - 1.0) * g.Rsp(n));
+    put(NT + NS + n, e_species(g, n, T, logT, Tinv));
+  }
+  im_branch_end();
+}
+
+// group G's species columns of a cell
+template <class M, int G>
+__device__ __forceinline__ void ijac_group(const ImArgs &a, double rho, double rhoinv, const double (&Y)[M::NS],
+                                           double *lds, int64_t code) {
+#pragma clang fp contract(off)
+  constexpr int NS = M::NS, NV = NS + 1, NT = sizeof(typename M::TCache) / sizeof(double);
+  constexpr int m0 = G * M::COLS, nm = NS - m0 < M::COLS ? NS - m0 : M::COLS;
+  const ImGroup X(a, lds);
+  double Yp[M::COLS] = {}, hd[M::COLS] = {}, omega[M::COLS + 1][NS];
+  const double h = *a.dt / a.parts;
+#pragma unroll
+  for (int c = 0; c < nm; c++) {
+    const double dlt = fd_step(Y[m0 + c], false);
+    Yp[c] = Y[m0 + c] + dlt;
+    hd[c] = h / dlt;
+  }
+  M::template fold_columns<G>(X.K, X.C, rho, Y, Yp, X, omega);
+  // dT/dt of a composition from its rates, rhs0d's sums
+  const auto dTdt = [&](int v) {
+    double cv = 0.0, d = 0.0;
+#pragma unroll
+    for (int n = 0; n < NS; n++) {
+      cv += X(NT + n) * (v && n == m0 + v - 1 ? Yp[v - 1] : Y[n]);
+      d -= X(NT + NS + n) * omega[v][n];
+    }
+    return d * (1.0 / (cv * rho));
+  };
+  double f0[NV];
+#pragma unroll
+  for (int r = 0; r < NS; r++) f0[r] = omega[0][r] * rhoinv;
+  f0[NS] = dTdt(0);
+  if constexpr (G == 0) {
+    double *fh = a.y + NV * a.ncell + code;
+#pragma unroll
+    for (int r = 0; r < NV; r++) fh[r * a.ncell] = f0[r];
+  }
+#pragma unroll
+  for (int c = 0; c < nm; c++) {
+    const int m = m0 + c;
+#pragma unroll
+    for (int r = 0; r < NS; r++)
+      a.A[a64_at<NV>(code, r, m)] = (r == m ? 1.0 : 0.0) - (omega[c + 1][r] * rhoinv - f0[r]) * hd[c];
+    a.A[a64_at<NV>(code, NS, m)] = 0.0 - (dTdt(c + 1) - f0[NS]) * hd[c];
+  }
+}
+
+// f<G>() for the wave's group, the last for any other wave; each ends its caller's path, as branches that
+// joined again would hold more
+template <int GROUPS, class F>
+__device__ __forceinline__ void im_group(int wave, F &&f) {
+  static_assert(GROUPS >= 1 && GROUPS <= 4);
+  if constexpr (GROUPS > 1)
+    if (wave == 0) return f.template operator()<0>();
+  if constexpr (GROUPS > 2)
+    if (wave == 1) return f.template operator()<1>();
+  if constexpr (GROUPS > 3)
+    if (wave == 2) return f.template operator()<2>();
+  if (wave == GROUPS - 1) return f.template operator()<GROUPS - 1>();
+}
+
+// a workgroup's species columns: lds im_cols_lds<M> bytes, the lane's cell (i, j, k) at work place code. A lane
+// past the cells takes the last one again, the same values to the same places: a branch around the stores
+// would cut the columns' one block in two, which the compiler then fills 512 registers between
 template <class M>
-__device__ __forceinline__ void ijac_base(const ImArgs &a, const View &Q, int i, int j, int k, int64_t code) {
+__device__ __forceinline__ void ijac_columns(const ImArgs &a, const View &Q, const View &st, double *lds, int i, int j,
+                                             int k, int64_t code) {
+#pragma clang fp contract(off)
+  constexpr int NS = M::NS, NV = NS + 1;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / IM_CELLS);
+  const int64_t o = Q.off(i, j, k);
+  const double rho = Q.at(o, 0), rhoinv = 1.0 / rho;
+  double y0[NV], Y[NS];
+  im_y0<M>(a, Q, st, o, st.off(i, j, k), rhoinv, code, y0);
+  if (wave == 0 && a.first) {
+#pragma unroll
+    for (int r = 0; r < NV; r++) a.y[r * a.ncell + code] = y0[r];
+  }
+  const double T = (double)(float)y0[NS];
+  im_group<M::GROUPS>(wave, [&]<int G>() { ijac_part<M, G>(a, T, lds); });
+  __syncthreads();
+#pragma unroll
+  for (int n = 0; n < NS; n++) Y[n] = (double)(float)y0[n];
+  im_group<M::GROUPS>(wave, [&]<int G>() { ijac_group<M, G>(a, rho, rhoinv, Y, lds, code); });
+}
+
+// slice 0: the T column of A by a whole evaluation; slice 1: f(y)
+template <class M>
+__device__ __forceinline__ void ijac_whole(const ImArgs &a, const View &Q, int i, int j, int k, int64_t code,
+                                           int slice) {
 #pragma clang fp contract(off)
   constexpr int NS = M::NS, NV = NS + 1;
   const int64_t nc = a.ncell;
   const double rho = Q.at(Q.off(i, j, k), 0), rhoinv = 1.0 / rho;
-  const double *y = a.y + code;
-  double yc[NV], fc[NV];
-#pragma unroll
-  for (int r = 0; r < NV; r++) yc[r] = (double)(float)y[r * nc];
-  ImCache<M> cc;
-  im_cache_load<M>(a.tc, nc, code, cc);
-  rhs0d_cached<M>(Gas<NS>{a.K}, a.C, rho, rhoinv, yc, cc, fc);
-  double *fh = a.y + NV * nc + code;
-#pragma unroll
-  for (int r = 0; r < NV; r++) fh[r * nc] = fc[r];
-}
-
-// slice m (wave-uniform) of the columns' launch: for m < ns + 1, column m of A, the rates at
-// y^ + dlt e_m less f(y^), over dlt, times -h, plus the identity's column; for m = ns + 1, f(y)
-template <class M>
-__device__ __forceinline__ void ijac_column(const ImArgs &a, const View &Q, int i, int j, int k, int64_t code,
-                                            int m) {
-#pragma clang fp contract(off)
-  constexpr int NS = M::NS, NV = NS + 1;
-  const int64_t nc = a.ncell;
-  const int64_t o = Q.off(i, j, k);
-  const double rho = Q.at(o, 0), rhoinv = 1.0 / rho;
   const double *y = a.y + code, *fh = a.y + NV * nc + code;
-  const bool column = m < NV;
-  double yp[NV], f1[NV], ym = 0.0;
+  double yp[NV], f1[NV];
 #pragma unroll
   for (int r = 0; r < NV; r++) {
     const double yr = y[r * nc];
-    yp[r] = column ? (double)(float)yr : yr;
-    ym = r == m ? yp[r] : ym;
+    yp[r] = slice == 0 ? (double)(float)yr : yr;
   }
-  const double dlt = fd_step(ym, m == NS);
-#pragma unroll
-  for (int r = 0; r < NV; r++) yp[r] = r == m ? ym + dlt : yp[r];
-  if (m < NS) {
-    // a species column: T is the base's, whose cache the base left
-    ImCache<M> cc;
-    im_cache_load<M>(a.tc, nc, code, cc);
-    rhs0d_cached<M>(Gas<NS>{a.K}, a.C, rho, rhoinv, yp, cc, f1);
-  } else {
-    rhs0d<M>(Gas<NS>{a.K}, a.C, rho, rhoinv, yp, f1);
-  }
-  if (!column) {
+  const double dlt = fd_step(yp[NS], true);
+  yp[NS] = slice == 0 ? yp[NS] + dlt : yp[NS];
+  rhs0d<M>(Gas<NS>{a.K}, a.C, rho, rhoinv, yp, f1);
+  if (slice == 1) {
     double *bv = a.y + 2 * NV * nc + code;
 #pragma unroll
     for (int r = 0; r < NV; r++) bv[r * nc] = f1[r];
     return;
   }
-  const double h = *a.dt / a.parts;
-  const double hd = h / dlt;
+  const double hd = *a.dt / a.parts / dlt;
 #pragma unroll
-  for (int r = 0; r < NV; r++) a.A[a64_at<NV>(code, r, m)] = (r == m ? 1.0 : 0.0) - (f1[r] - fh[r * nc]) * hd;
+  for (int r = 0; r < NV; r++) a.A[a64_at<NV>(code, r, NS)] = (r == NS ? 1.0 : 0.0) - (f1[r] - fh[r * nc]) * hd;
 }
 
 // what a slice of the columns' launch leaves for a work place that holds no cell (a tile's overhang in
@@ -590,28 +629,21 @@ __device__ __forceinline__ void iend_cell(const ImArgs &a, const View &Q, const 
 }
 
 template <class M>
-__global__ __launch_bounds__(FLAT) void k_itc(ImArgs a) {
+__global__ __launch_bounds__(M::GROUPS *IM_CELLS) void k_icol(ImArgs a) {
+  extern __shared__ double lds[];
+  const unsigned c = min(xcd_block() * IM_CELLS + threadIdx.x % IM_CELLS, (unsigned)a.ncell - 1);
   int i, j, k;
-  if (!flat_cell_of(a.b, i, j, k)) return;
-  ijac_tcache<M>(a, a.Q, a.st, i, j, k, im_code(a.b, i, j, k));
+  cell_at(a.b, c, i, j, k);
+  ijac_columns<M>(a, a.Q, a.st, lds, i, j, k, c);
 }
 
+// a tile's two slices in workgroups numbered one after another, so one XCD's L2 serves y to both
 template <class M>
-__global__ __launch_bounds__(FLAT) void k_ibase(ImArgs a) {
+__global__ __launch_bounds__(FLAT) void k_iwhole(ImArgs a) {
+  const unsigned g = xcd_block();
   int i, j, k;
-  if (!flat_cell_of(a.b, i, j, k)) return;
-  ijac_base<M>(a, a.Q, i, j, k, im_code(a.b, i, j, k));
-}
-
-// every slice of a tile of cells (the ns + 1 columns and f(y)) in workgroups numbered one after
-// another, so one XCD runs a tile's slices and its L2 serves y and f(y^) to all of them
-template <class M>
-__global__ __launch_bounds__(FLAT) void k_icol(ImArgs a) {
-  constexpr unsigned S = M::NS + 2;
-  const unsigned g = xcd_block(), tile = g / S;
-  int i, j, k;
-  if (!flat_at(a.b, tile, i, j, k)) return;
-  ijac_column<M>(a, a.Q, i, j, k, im_code(a.b, i, j, k), (int)(g - tile * S));
+  if (!flat_at(a.b, g / 2, i, j, k)) return;
+  ijac_whole<M>(a, a.Q, i, j, k, im_code(a.b, i, j, k), (int)(g % 2));
 }
 
 // four waves of 16 cells per workgroup

@@ -144,10 +144,6 @@ inline Turn turn_of(const double *R) {
 #define PGA_REALGAS_CASES(ns) ((ns) == 1 || (ns) == 2)
 #endif
 
-// doubles of a cell's cache of the implicit chemistry's f at one T for the case's mechanism, -1 for
-// none (pga_implicit.hip)
-int64_t im_cache_doubles(const pga_case_desc &d);
-
 // the species counts the cubic real gas is compiled for (its kernels are the heaviest to build)
 constexpr bool realgas_compiled(int ns) { return PGA_REALGAS_CASES(ns); }
 

@@ -166,11 +166,11 @@ def render(name, records, sets, ns):
     w("  __device__ __forceinline__ static void fold(const double *__restrict__ C, const Rates &s, double (&omega)[NS],")
     w("                                              double (&D)[NS]) {")
     _fold_prologue(w, L, records, ns, logform, product)
-    _fold_reactions(w, L, records, cached=False)
+    _fold_reactions(w, L, records)
     w("  }")
     # what the rates at one T share whatever the composition, for the forward-difference columns of
     # implicit chemistry (a species column changes the composition at the same T): each value is the
-    # expression ratestate and fold evaluate, so cstate + fold_cached give fold's bits
+    # expression ratestate and fold evaluate, so tstate_part + fold_columns give fold's bits
     w(f"  static constexpr int NX = {len(records)};")
     w("  struct TCache {")
     w("    double logT, Tinv;")
@@ -180,9 +180,6 @@ def render(name, records, sets, ns):
         w(f"    double prefRuT, prefRuTinv, eG[{ns}];")
     w(f"    double gRT[{ns}], kx[{len(records)}];")
     w("  };")
-    # tstate stores each value where TCache's member lies (out[index * stride]) as soon as it is
-    # made: with C and out in one restrict scope the constants keep their scalar loads and no value
-    # waits in a register for the others
     off = {"logT": 0, "Tinv": 1}
     at = 2
     if logform:
@@ -193,77 +190,8 @@ def render(name, records, sets, ns):
         at += 2 + ns
     off["gRT"] = at
     off["kx"] = at + ns
-    w("  __device__ __forceinline__ static void tstate(const Gas<NS> &g, const double *__restrict__ C, double T,")
-    w("                                                double *__restrict__ out, long long stride) {")
-    w("#pragma clang fp contract(off)")
-    w("    const double logT = tlog(T), Tinv = 1.0 / T;")
-    w(f"    out[{off['logT']} * stride] = logT;")
-    w(f"    out[{off['Tinv']} * stride] = Tinv;")
-    if logform:
-        w(f"    out[{off['logprefRuT']} * stride] = C[{L.scalar('logprefRu')}] - logT;")
-    if product:
-        w(f"    out[{off['prefRuT']} * stride] = C[{L.scalar('prefRu')}] * Tinv;")
-        w(f"    out[{off['prefRuTinv']} * stride] = C[{L.scalar('Rupref')}] * T;")
-    w(f"    double gRT[{ns}];")
-    w("#pragma unroll")
-    w(f"    for (int n = 0; n < {ns}; n++) {{")
-    w("      gRT[n] = gibbs_rt(g, n, logT, Tinv);")
-    w(f"      out[({off['gRT']} + n) * stride] = gRT[n];")
-    if product:
-        w(f"      out[({off['eG']} + n) * stride] = texp(gRT[n]);")
-    w("    }")
-    w(f"    const double expclamp = C[{L.scalar('expclamp')}];")
-    w("    (void)expclamp;")
-    for k, r in enumerate(records):
-        kind = _cached(r)
-        dest = f"out[{off['kx'] + k} * stride]"
-        if kind is None:
-            w(f"    {dest} = 0.0;")
-            continue
-        w(f"    {{  // reaction {k}: {kind}")
-        if kind == "lfc":
-            _troe_lfc(w, L, r, into=dest)
-        else:
-            _arrhenius(w, L, k, r)
-            if kind == "lk":
-                w(f"      {dest} = lk;")
-            else:
-                w("      double xk = lk;")
-                for j, (sp, _) in enumerate(r.react):
-                    w(f"      xk -= C[{L.listed(k, 'reactnu', j)}] * gRT[{sp}];")
-                w(f"      {dest} = texp(fmin(xk, expclamp));")
-        w("    }")
-    w("  }")
-    w("  __device__ __forceinline__ static void cstate(const Gas<NS> &g, const double *__restrict__ C, double rho,")
-    w("                                                const double (&Y)[NS], const TCache &t, Rates &s) {")
-    w("#pragma clang fp contract(off)")
-    w("    s.logT = t.logT;")
-    w("    s.Tinv = t.Tinv;")
-    if logform:
-        w("    s.logprefRuT = t.logprefRuT;")
-    if product:
-        w("    s.prefRuT = t.prefRuT;")
-        w("    s.prefRuTinv = t.prefRuTinv;")
-    w("    double ctot = 0.0;")
-    w("#pragma unroll")
-    w(f"    for (int n = 0; n < {ns}; n++) {{")
-    w("      const double c = rho * Y[n] * g.MWinv(n);")
-    w("      ctot += c;")
-    w("      s.gRT[n] = t.gRT[n];")
-    if logform:
-        w(f"      s.logc[n] = fmax(C[{L.scalar('logcfloor')}], tlog(c));")
-    if product:
-        w("      s.cG[n] = fmax(c, 0.0) * t.eG[n];")
-    w("    }")
-    w("    s.ctot = ctot;")
-    _ctb(w, L, sets, plainbodies, logbodies)
-    w("  }")
-    w("  template <bool WITHD>")
-    w("  __device__ __forceinline__ static void fold_cached(const double *__restrict__ C, const Rates &s,")
-    w("                                                     const TCache &t, double (&omega)[NS], double (&D)[NS]) {")
-    _fold_prologue(w, L, records, ns, logform, product)
-    _fold_reactions(w, L, records, cached=True)
-    w("  }")
+    _tstate_part(w, L, records, ns, off, logform, product)
+    _fold_columns(w, L, records, sets, ns, off, logform, product)
     w("  __device__ __forceinline__ static void production(const Gas<NS> &g, const double *__restrict__ C,")
     w("                                                    double rho, const double (&Y)[NS], double T, double (&omega)[NS]) {")
     w("    Rates s;")
@@ -320,72 +248,96 @@ def _arrhenius(w, L, k, r):
         w(f"      lk -= C[{L.field(k, 'EaR')}] * Tinv;")
 
 
-def _fold_reactions(w, L, records, cached):
-    """The fold's reactions (finiterate.mako:185-236); cached: the T-only values (_cached) read
-    from the TCache t rather than evaluated, each the same expression in the same order."""
-    for k, r in enumerate(records):
-        w(f"    {{  // reaction {k}: {r.equation} ({r.name}{', reversible' if r.reversible else ''}, {'product' if r.product else 'log'} form)")
-        kind = _cached(r) if cached else None
-        if kind == "lk":
-            w(f"      double lk = t.kx[{k}];")
-        elif kind != "K":
-            _arrhenius(w, L, k, r)
-        if r.product:
-            if r.falloff:
-                _logpr(w, L, k, r)
-                w("      const double pr = texp(fmin(logpr, expclamp));")
-                w("      const double pfac = pr / (1.0 + pr);")
-            if r.troe:
-                _troe_lfc(w, L, r) if kind != "lfc" else w(f"      const double lfc = t.kx[{k}];")
-                _troe_use(w)
-            if kind == "K":
-                w(f"      double K = t.kx[{k}];")
-            else:
-                w("      double xk = lk;")
-                for j, (sp, _) in enumerate(r.react):
-                    w(f"      xk -= C[{L.listed(k, 'reactnu', j)}] * s.gRT[{sp}];")
-                w("      double K = texp(fmin(xk, expclamp));")
-            if r.thirdbody and not r.falloff:
-                w(f"      K *= s.ctb[{r.tb}];")
-            if r.falloff:
-                w("      K *= pfac;")
-            w("      double fwd = K;")
-            for sp, nu in r.react:
+class _Names:
+    """What a reaction's rate is written in: the rate state s."""
+
+    def cG(self, sp):
+        return f"s.cG[{sp}]"
+
+    def logc(self, sp):
+        return f"s.logc[{sp}]"
+
+    def gRT(self, sp):
+        return f"s.gRT[{sp}]"
+
+    def ctb(self, j):
+        return f"s.ctb[{j}]"
+
+    def logtb(self, j):
+        return f"s.logtb[{j}]"
+
+
+def _reaction_rate(w, L, k, r, kind, x):
+    """fwd, rev and rp of reaction k; kind: its T-only value (_cached) read rather than evaluated, each
+    the same expression in the same order."""
+    if kind == "lk":
+        w(f"      double lk = {x.kx(k)};")
+    elif kind != "K":
+        _arrhenius(w, L, k, r)
+    if r.product:
+        if r.falloff:
+            _logpr(w, L, k, r, x)
+            w("      const double pr = texp(fmin(logpr, expclamp));")
+            w("      const double pfac = pr / (1.0 + pr);")
+        if r.troe:
+            _troe_lfc(w, L, r) if kind != "lfc" else w(f"      const double lfc = {x.kx(k)};")
+            _troe_use(w)
+        if kind == "K":
+            w(f"      double K = {x.kx(k)};")
+        else:
+            w("      double xk = lk;")
+            for j, (sp, _) in enumerate(r.react):
+                w(f"      xk -= C[{L.listed(k, 'reactnu', j)}] * {x.gRT(sp)};")
+            w("      double K = texp(fmin(xk, expclamp));")
+        if r.thirdbody and not r.falloff:
+            w(f"      K *= {x.ctb(r.tb)};")
+        if r.falloff:
+            w("      K *= pfac;")
+        w("      double fwd = K;")
+        for sp, nu in r.react:
+            for _ in range(int(nu)):
+                w(f"      fwd *= {x.cG(sp)};")
+        if r.reversible:
+            w("      double rev = K;")
+            for _ in range(int(abs(r.nusum))):
+                w(f"      rev *= {'prefRuTinv' if r.nusum > 0 else 'prefRuT'};")
+            for sp, nu in r.prod:
                 for _ in range(int(nu)):
-                    w(f"      fwd *= s.cG[{sp}];")
-            if r.reversible:
-                w("      double rev = K;")
-                for _ in range(int(abs(r.nusum))):
-                    w(f"      rev *= {'prefRuTinv' if r.nusum > 0 else 'prefRuT'};")
-                for sp, nu in r.prod:
-                    for _ in range(int(nu)):
-                        w(f"      rev *= s.cG[{sp}];")
-            else:
-                w("      const double rev = 0.0;")
+                    w(f"      rev *= {x.cG(sp)};")
+        else:
+            w("      const double rev = 0.0;")
+        w("      const double rp = fwd - rev;")
+    else:
+        if r.thirdbody and not r.falloff:
+            w(f"      lk += {x.logtb(r.tb)};")
+        if r.falloff:
+            _logpr(w, L, k, r, x)
+            w("      const double prexp = texp(-fabs(logpr));")
+            w("      lk += fmin(logpr, 0.0) - dlog1p(prexp);")
+        if r.troe:
+            _troe_lfc(w, L, r) if kind != "lfc" else w(f"      const double lfc = {x.kx(k)};")
+            _troe_use(w)
+        w("      double lrp = lk;")
+        for j, (sp, _) in enumerate(r.fwd):
+            w(f"      lrp += C[{L.listed(k, 'fwdorder', j)}] * {x.logc(sp)};")
+        if r.reversible:
+            first = f"C[{L.field(k, 'nusum')}] * logprefRuT" if r.nusum != 0.0 else "0.0"
+            w(f"      double diff = {first};")
+            for j, (sp, _, _) in enumerate(r.net):
+                w(f"      diff -= C[{L.listed(k, 'netnu', j)}] * ({x.gRT(sp)} + {x.logc(sp)});")
+            w("      const double fwd = texp(fmin(lrp, expclamp)), rev = texp(fmin(lrp - diff, expclamp));")
             w("      const double rp = fwd - rev;")
         else:
-            if r.thirdbody and not r.falloff:
-                w(f"      lk += s.logtb[{r.tb}];")
-            if r.falloff:
-                _logpr(w, L, k, r)
-                w("      const double prexp = texp(-fabs(logpr));")
-                w("      lk += fmin(logpr, 0.0) - dlog1p(prexp);")
-            if r.troe:
-                _troe_lfc(w, L, r) if kind != "lfc" else w(f"      const double lfc = t.kx[{k}];")
-                _troe_use(w)
-            w("      double lrp = lk;")
-            for j, (sp, _) in enumerate(r.fwd):
-                w(f"      lrp += C[{L.listed(k, 'fwdorder', j)}] * s.logc[{sp}];")
-            if r.reversible:
-                first = f"C[{L.field(k, 'nusum')}] * logprefRuT" if r.nusum != 0.0 else "0.0"
-                w(f"      double diff = {first};")
-                for j, (sp, _, _) in enumerate(r.net):
-                    w(f"      diff -= C[{L.listed(k, 'netnu', j)}] * (s.gRT[{sp}] + s.logc[{sp}]);")
-                w("      const double fwd = texp(fmin(lrp, expclamp)), rev = texp(fmin(lrp - diff, expclamp));")
-                w("      const double rp = fwd - rev;")
-            else:
-                w("      const double fwd = texp(fmin(lrp, expclamp)), rev = 0.0;")
-                w("      const double rp = fwd;")
+            w("      const double fwd = texp(fmin(lrp, expclamp)), rev = 0.0;")
+            w("      const double rp = fwd;")
+
+
+def _fold_reactions(w, L, records):
+    """The fold's reactions (finiterate.mako:185-236)."""
+    x = _Names()
+    for k, r in enumerate(records):
+        w(f"    {{  // reaction {k}: {r.equation} ({r.name}{', reversible' if r.reversible else ''}, {'product' if r.product else 'log'} form)")
+        _reaction_rate(w, L, k, r, None, x)
         for j, (sp, _, nuMW) in enumerate(r.net):
             w(f"      omega[{sp}] += C[{L.listed(k, 'netnuMW', j)}] * rp;")
         w("      if constexpr (WITHD) {")
@@ -398,8 +350,174 @@ def _fold_reactions(w, L, records, cached):
         w("    }")
 
 
-def _logpr(w, L, k, r):
-    w(f"      double logpr = s.logtb[{r.tb}] + C[{L.field(k, 'logprA')}];")
+class _ColumnNames(_Names):
+    """Column v >= 1 of a group, its (v - 1)-th species moved (v = 0: the base): the moved species' values are
+    the column's own, the others the base's."""
+
+    def __init__(self, v, moved, off):
+        self.v, self.moved, self.off = v, moved, off
+
+    def of(self, name, sp):
+        return f"{name}{sp}_{self.v}" if self.v and sp == self.moved else f"{name}{sp}_0"
+
+    def cG(self, sp):
+        return self.of("cG", sp)
+
+    def logc(self, sp):
+        return self.of("logc", sp)
+
+    def gRT(self, sp):
+        return f"X({self.off['gRT'] + sp})"
+
+    def ctb(self, j):
+        return f"ctb{j}_{self.v}"
+
+    def logtb(self, j):
+        return f"logtb{j}_{self.v}"
+
+    def kx(self, k):
+        return f"X({self.off['kx'] + k})"
+
+
+# the species columns a lane takes beside the base (implicit chemistry's workgroups have a wave a group)
+COLUMNS = 3
+
+
+def _touches(r, sp):
+    """Whether the reaction's rate changes with species sp alone at one T."""
+    if r.thirdbody or r.falloff:
+        return True
+    if r.product:
+        return any(s == sp for s, _ in r.react) or (r.reversible and any(s == sp for s, _ in r.prod))
+    return any(s == sp for s, _ in r.fwd) or (r.reversible and any(s == sp for s, _, _ in r.net))
+
+
+def _tstate_part(w, L, records, ns, off, logform, product):
+    """One of GROUPS shares of the TCache at T, each value put (put(index, value)) where TCache's member lies."""
+    groups = -(-ns // COLUMNS)
+    w(f"  static constexpr int COLS = {COLUMNS}, GROUPS = {groups};")
+    w("  template <int G, class GA, class PUT>")
+    w("  __device__ __forceinline__ static void tstate_part(const GA &g, Constants C, double T, const PUT &put) {")
+    w("#pragma clang fp contract(off)")
+    w("    const double logT = tlog(T), Tinv = 1.0 / T;")
+    w(f"    double gRT[{ns}];")
+    w("#pragma unroll")
+    w(f"    for (int n = 0; n < {ns}; n++) gRT[n] = gibbs_rt(g, n, logT, Tinv);")
+    w(f"    const double expclamp = C[{L.scalar('expclamp')}];")
+    w("    (void)expclamp;")
+    for G in range(groups):
+        w(f"    if constexpr (G == {G}) {{")
+        if G == 0:
+            w(f"    put({off['logT']}, logT);")
+            w(f"    put({off['Tinv']}, Tinv);")
+            if logform:
+                w(f"    put({off['logprefRuT']}, C[{L.scalar('logprefRu')}] - logT);")
+            if product:
+                w(f"    put({off['prefRuT']}, C[{L.scalar('prefRu')}] * Tinv);")
+                w(f"    put({off['prefRuTinv']}, C[{L.scalar('Rupref')}] * T);")
+        for n in range(G, ns, groups):
+            w(f"    put({off['gRT'] + n}, gRT[{n}]);")
+            if product:
+                w(f"    put({off['eG'] + n}, texp(gRT[{n}]));")
+        for k, r in list(enumerate(records))[G::groups]:
+            kind = _cached(r)
+            at = off["kx"] + k
+            if kind is None:
+                w(f"    put({at}, 0.0);")
+                continue
+            w(f"    {{  // reaction {k}: {kind}")
+            if kind == "lfc":
+                _troe_lfc(w, L, r)
+                w(f"      put({at}, lfc);")
+            else:
+                _arrhenius(w, L, k, r)
+                if kind == "lk":
+                    w(f"      put({at}, lk);")
+                else:
+                    w("      double xk = lk;")
+                    for j, (sp, _) in enumerate(r.react):
+                        w(f"      xk -= C[{L.listed(k, 'reactnu', j)}] * gRT[{sp}];")
+                    w(f"      put({at}, texp(fmin(xk, expclamp)));")
+            w("    }")
+        w("    }")
+    w("  }")
+
+
+def _fold_columns(w, L, records, sets, ns, off, logform, product):
+    """The rates at one T of a base composition, omega[0], and with one species moved for each of a group's
+    COLUMNS species: cstate + fold_cached's values of each, a reaction's rate evaluated again only for the
+    columns whose species it reads."""
+    w("  template <int G, class TC>")
+    w("  __device__ __forceinline__ static void fold_columns(Constants K, Constants C, double rho,")
+    w("                                                      const double (&Y)[NS], const double (&Yp)[COLS], const TC &X,")
+    w("                                                      double (&omega)[COLS + 1][NS]) {")
+    w("    // one rounding per written operation, as the oracle evaluates the fold")
+    w("#pragma clang fp contract(off)")
+    w(f"    const double logT = X({off['logT']}), Tinv = X({off['Tinv']});")
+    w("    (void)logT, (void)Tinv;")
+    if logform:
+        w(f"    const double logprefRuT = X({off['logprefRuT']});")
+        w("    (void)logprefRuT;")
+    if product:
+        w(f"    const double prefRuT = X({off['prefRuT']}), prefRuTinv = X({off['prefRuTinv']});")
+        w("    (void)prefRuT, (void)prefRuTinv;")
+    w(f"    const double expclamp = C[{L.scalar('expclamp')}];")
+    w("    (void)expclamp;")
+    if any(r.troe for r in records):
+        w("    const double log10e = 0.4342944819032518, ln10 = 2.302585092994046;")
+    w("#pragma unroll")
+    w("    for (int v = 0; v <= COLS; v++)")
+    w("#pragma unroll")
+    w(f"      for (int n = 0; n < {ns}; n++) omega[v][n] = 0.0;")
+
+    def species(n, v, y):
+        w(f"    const double c{n}_{v} = rho * {y} * K[Gas<NS>::O.MWinv + {n}];")
+        if product:
+            w(f"    const double cG{n}_{v} = fmax(c{n}_{v}, 0.0) * X({off['eG'] + n});")
+        if logform:
+            w(f"    const double logc{n}_{v} = fmax(C[{L.scalar('logcfloor')}], tlog(c{n}_{v}));")
+
+    for n in range(ns):
+        species(n, 0, f"Y[{n}]")
+    for G in range(-(-ns // COLUMNS)):
+        moved = list(range(G * COLUMNS, min(ns, (G + 1) * COLUMNS)))
+        w(f"    if constexpr (G == {G}) {{  // species {moved[0]} to {moved[-1]}")
+        for v, m in enumerate(moved, 1):
+            species(m, v, f"Yp[{v - 1}]")
+        cols = [_ColumnNames(0, -1, off)] + [_ColumnNames(v, m, off) for v, m in enumerate(moved, 1)]
+        for x in cols:
+            w(f"    double ctot_{x.v} = 0.0;")
+            for n in range(ns):
+                w(f"    ctot_{x.v} += {x.of('c', n)};")
+        summed, logged = set(), set()
+        for k, r in enumerate(records):
+            if r.thirdbody or r.falloff:
+                # a third body's sums, made where a reaction first reads them
+                for x in cols:
+                    if r.tb not in summed:
+                        w(f"    double ctb{r.tb}_{x.v} = C[{L.tbdefeff(r.tb)}] * ctot_{x.v};")
+                        for e, (sp, _) in enumerate(sets[r.tb].eff):
+                            w(f"    ctb{r.tb}_{x.v} += C[{L.tbeffdev(r.tb, e)}] * {x.of('c', sp)};")
+                    if (r.falloff or not r.product) and r.tb not in logged:
+                        w(f"    const double logtb{r.tb}_{x.v} = tlog(fmax(2.2250738585072014e-308, ctb{r.tb}_{x.v}));")
+                summed.add(r.tb)
+                if r.falloff or not r.product:
+                    logged.add(r.tb)
+            own = [x for x in cols[1:] if _touches(r, x.moved)]
+            for x, takers in [(cols[0], [y for y in cols if y not in own])] + [(x, [x]) for x in own]:
+                w(f"    {{  // reaction {k}: {r.equation}")
+                _reaction_rate(w, L, k, r, _cached(r), x)
+                for y in takers:
+                    for j, (sp, _, _) in enumerate(r.net):
+                        w(f"      omega[{y.v}][{sp}] += C[{L.listed(k, 'netnuMW', j)}] * rp;")
+                w("      (void)rev;")
+                w("    }")
+        w("    }")
+    w("  }")
+
+
+def _logpr(w, L, k, r, x):
+    w(f"      double logpr = {x.logtb(r.tb)} + C[{L.field(k, 'logprA')}];")
     if r.prb != 0.0:
         w(f"      logpr += C[{L.field(k, 'prb')}] * logT;")
     if r.prEaR != 0.0:
