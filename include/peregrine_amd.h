@@ -399,7 +399,7 @@ int64_t pga_implicit_worksize(const pga_case *c, pga_box box);
  * same 0D system the sub-stepped form does (its ns mass fractions and T at constant density and
  * internal energy, chemint/kernels/substep.mako:14-50) by the linearly implicit Euler method in
  * o->parts parts, y1 = y0 + h x with (I - h J) x = f(y0), J by forward differences in FP64. Each
- * matrix is factored in FP32 on the matrix cores, 16 cells per wave, and in the same registers
+ * matrix is factored in FP32, a lane per cell, and in the same registers
  * each solve is refined against the FP64 matrix with FP64 residuals until every row's residual is
  * within o->tolerance of its scale |f_i| + sum_j |A_ij x_j|. It writes the mean rate over the step, rho (Y_end - Y_start) / dt,
  * into dQ (rows 0..4 zero) when begin_dQ, else into the ns - 1 rows of `out` as pga_rates does, and

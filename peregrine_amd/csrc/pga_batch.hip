@@ -565,14 +565,14 @@ extern "C" int32_t pga_batch_implicit(const pga_batch *h, const pga_implicit_opt
   bool done = false;
 #define X(NAME, IDX)                                                                             \
   if (d.mechanism == IDX) {                                                                      \
-    constexpr int NV = Mech_##NAME::NS + 1, NB = (NV + 3) / 4;                                   \
+    constexpr int NV = Mech_##NAME::NS + 1;                                                      \
     hipLaunchKernelGGL((kb_ivoid<NV>), grid, dim3(FLAT), 0, s, a, im);                           \
     for (int part = 0; part < o->parts; part++) {                                                \
       im.first = part == 0, im.last = part == o->parts - 1;                                      \
       hipLaunchKernelGGL((kb_icol<Mech_##NAME>), dim3(grid.x * (FLAT / IM_CELLS)),               \
                          dim3(Mech_##NAME::GROUPS * IM_CELLS), im_cols_lds<Mech_##NAME>, s, a, im); \
       hipLaunchKernelGGL((kb_iwhole<Mech_##NAME>), dim3(grid.x * 2), dim3(FLAT), 0, s, a, im);   \
-      hipLaunchKernelGGL((k_lusolve<NB, NV>), dim3((unsigned)((groups + 3) / 4)), dim3(256), 0, s, im); \
+      hipLaunchKernelGGL((k_lusolve<NV>), dim3((unsigned)((cells + 63) / 64)), dim3(64), 0, s, im); \
     }                                                                                            \
     hipLaunchKernelGGL((kb_iend<Mech_##NAME>), grid, dim3(FLAT), 0, s, a, im);                  \
     done = true;                                                                                 \

@@ -1,5 +1,5 @@
 // Implicit chemistry's entry points (the kernels are in pga_implicit.hpp): per part of the step,
-// the forward-difference matrices, their batched FP32 LU on the matrix cores, and the refined
+// the forward-difference matrices, their FP32 LU, and the refined
 // linearly implicit step; and the batched solve of caller-given systems.
 #include "pga_implicit.hpp"
 #include "pga_internal.hpp"
@@ -97,13 +97,13 @@ extern "C" int32_t pga_implicit(const pga_case *c, const pga_implicit_opts *o, p
   bool done = false;
 #define X(NAME, IDX)                                                                              \
   if (d.mechanism == IDX) {                                                                       \
-    constexpr int NV = Mech_##NAME::NS + 1, NB = (NV + 3) / 4;                                    \
+    constexpr int NV = Mech_##NAME::NS + 1;                                                       \
     for (int part = 0; part < o->parts; part++) {                                                 \
       a.first = part == 0, a.last = part == o->parts - 1;                                         \
       hipLaunchKernelGGL((k_icol<Mech_##NAME>), dim3((unsigned)((cells + IM_CELLS - 1) / IM_CELLS)), \
                          dim3(Mech_##NAME::GROUPS * IM_CELLS), im_cols_lds<Mech_##NAME>, s, a);   \
       hipLaunchKernelGGL((k_iwhole<Mech_##NAME>), dim3(grid.x * 2), dim3(FLAT), 0, s, a);        \
-      hipLaunchKernelGGL((k_lusolve<NB, NV>), dim3((unsigned)((groups + 3) / 4)), dim3(256), 0, s, a); \
+      hipLaunchKernelGGL((k_lusolve<NV>), dim3((unsigned)((cells + 63) / 64)), dim3(64), 0, s, a); \
     }                                                                                             \
     hipLaunchKernelGGL((k_iend<Mech_##NAME>), grid, dim3(FLAT), 0, s, a);                        \
     done = true;                                                                                  \

@@ -8,28 +8,27 @@
 // A part of length h from y0 = (Y_0 .. Y_{ns-1}, T) takes y1 = y0 + h x with (I - h J) x = f(y0):
 // backward Euler's first Newton step, first order and stable however stiff the chemistry. J is
 // formed in FP64 by forward differences of f (one more evaluation of the rates per unknown); the
-// matrix is kept in FP64 and, rounded to FP32, factored by a batched LU on the matrix cores. The
+// matrix is kept in FP64 and, rounded to FP32, factored in registers. The
 // solve is an iterative refinement: x += (LU)^-1 r with the residual r = f - A x taken in FP64
 // against the FP64 matrix, until every row's residual is within `tolerance` of that row's scale
 // (|f_i| + sum_j |A_ij x_j|, the componentwise backward error), so x is the FP64 solution whatever
 // the factors' rounding. The Arrhenius exponentials, the Gibbs polynomials, the residuals and the
-// update stay FP64.
+// update stay FP64. No pivoting: the matrices are I - h J of a chemical source, whose diagonal grows with
+// the destruction rates; the FP64 refinement corrects what the FP32 factors leave.
 //
-// The batched LU takes 16 matrices per wave, padded to 12 x 12 (three 4 x 4 blocks a side), one
-// lane quad per matrix: lane 4b + q holds column q of each of matrix b's blocks, a block's row i in
-// its register i. That is the accumulator layout of v_mfma_f32_4x4x1f32 (16 independent 4 x 4
+// The batched LU of caller-given systems takes 16 matrices per wave, padded to 12 x 12 (three 4 x 4 blocks a
+// side), one lane quad per matrix: lane 4b + q holds column q of each of matrix b's blocks, a block's row i
+// in its register i. That is the accumulator layout of v_mfma_f32_4x4x1f32 (16 independent 4 x 4
 // products per instruction), so the Schur-complement updates of the blocked right-looking LU,
 // A_IJ -= L_IK U_KJ, are four rank-one MFMAs each for all 16 matrices at once; the diagonal blocks'
 // factorisation and the two triangular block solves run on the VALU within the quad, with DPP
-// broadcasts. No pivoting: the matrices are I - h J of a chemical source, whose diagonal grows with
-// the destruction rates; the FP64 refinement corrects what the FP32 factors leave.
+// broadcasts.
 //
 // The implicit form's work array holds the FP64 matrices, [group of 16 cells][(ns + 1)^2 entries]
-// [16 cells] (a row of the 16 cells' same entry is 128 contiguous bytes, so both the lane-per-cell
-// kernels and the quad-per-cell solve move whole segments), then y, f at y's FP32 rounding and f at
-// y, [ns + 1][cells] doubles each. The FP32 factors never leave the registers of the solve. The
-// batched solve of caller-given systems keeps its FP32 factors in a work array the same way,
-// [group][144 entries][16 cells].
+// [16 cells] (a row of the 16 cells' same entry is 128 contiguous bytes, so the lane-per-cell
+// kernels move whole segments), then y, f at y's FP32 rounding and f at y, [ns + 1][cells] doubles each.
+// The FP32 factors never leave the registers of the solve. The batched solve of caller-given systems
+// keeps its FP32 factors in a work array the same way, [group][144 entries][16 cells].
 #pragma once
 
 #include <type_traits>
@@ -64,22 +63,6 @@ __host__ __device__ __forceinline__ void sfor(F &&f) {
 template <int P>
 __device__ __forceinline__ float qb(float x) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), P * 0x55, 0xf, 0xf, false));
-}
-
-// a double moved within each quad: lane q takes lane PERM's pick of the quad (DPP quad_perm on both
-// halves; 0xB1 swaps neighbours, 0x4E swaps pairs)
-template <int PERM>
-__device__ __forceinline__ double qperm(double x) {
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), PERM, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), PERM, 0xf, 0xf, false);
-  return __hiloint2double(hi, lo);
-}
-
-// the sum of x over the quad, the same bits on its four lanes ((x0 + x1) + (x2 + x3), each add
-// commuted alike)
-__device__ __forceinline__ double qsum(double x) {
-  const double s = x + qperm<0xB1>(x);
-  return s + qperm<0x4E>(s);
 }
 
 // The blocked LU of one lane quad's matrix per quad, 16 per wave, in registers: lane q holds column q
@@ -499,108 +482,75 @@ __device__ __forceinline__ void ijac_void(const ImArgs &a, int64_t code, int m) 
   }
 }
 
-// The part's solve and step, a lane quad per cell, 16 cells per wave: (I - h J) x = f(y) by iterative
-// refinement, then y += h x. The quad loads its FP64 matrix once (lane q: columns q, q + 4, q + 8)
-// and keeps it, and the FP32 factors of its rounding (lu_factor), in registers; each sweep solves
-// L U z = r in FP32 with the residual broadcast to the quad, adds z to x and takes r = f - A x in
-// FP64 (each lane's columns, summed over the quad) with the row scales |f_m| + sum_c |A_mc x_c|. A
-// cell stops when every row's residual is within tol of its scale (its x then stays as it is), or
-// after maxsweeps; the wave runs until its last cell stops. Lane q keeps rows q, q + 4, q + 8 of x, f
-// and r. A cell's x depends only on its own matrix and f, whichever cells share its wave.
-template <int NB, int NV>
-__device__ __forceinline__ void lu_refine_group(const ImArgs &a, int64_t grp, int lane) {
+// The part's solve and step, a lane per cell: (I - h J) x = f(y) by iterative refinement, then y += h x. The
+// lane loads its FP64 matrix once and keeps it, and the FP32 factors of its rounding, in registers, at one
+// wave a SIMD; each sweep solves L U z = r in FP32, adds z to x and takes r = f - A x in FP64 with the row
+// scales |f_m| + sum_c |A_mc x_c|. A cell stops when every row's residual is within tol of its scale, or
+// after maxsweeps. A cell's x depends only on its own matrix and f, whichever cells share its wave.
+//
+// A quad of lanes per cell, with the matrix cores' rank-one updates between the quads' broadcasts, took 2150
+// vector instructions for 16 cells where this takes some 2500 for 64, each triangular solve a chain four lanes
+// share: 106 us for 64^3 cells, 60 here, 3.6 TB/s of the matrices' and vectors' bytes (the same factors, sums
+// and x to the bit). The 381 registers a lane holds leave one wave a SIMD; read again each sweep instead, the
+// matrices would be three passes over HBM.
+//
+// The sums go column c into the (c mod 4)-th of four partial sums, then ((0) + (1)) + ((2) + (3)).
+template <int NV>
+__device__ __forceinline__ void lu_refine_cell(const ImArgs &a, int64_t cell) {
 #pragma clang fp contract(off)
-  const int b = lane >> 2, q = lane & 3;
-  const int64_t nc = a.ncell, cell = grp * IM_G + b;
-  const bool real = cell < nc;
-  const int64_t at = real ? cell : grp * IM_G;
-  double Ad[NB][NV];
-  sfor<0, NB>([&]<int J>() {
-    const int c = 4 * J + q;
-    const int cc = c < NV ? c : 0;
-    sfor<0, NV>([&]<int m>() {
-      const double v = a.A[a64_at<NV>(at, m, cc)];
-      Ad[J][m] = !real ? (m == c ? 1.0 : 0.0) : (c < NV ? v : 0.0);
+  const int64_t nc = a.ncell;
+  const double *A = a.A + a64_at<NV>(cell, 0, 0), *bvp = a.y + 2 * NV * nc + cell;
+  double Ad[NV][NV], bv[NV], x[NV], r[NV];
+  sfor<0, NV>([&]<int m>() { sfor<0, NV>([&]<int c>() { Ad[m][c] = A[(m * NV + c) * IM_G]; }); });
+  sfor<0, NV>([&]<int m>() { bv[m] = bvp[m * nc]; });
+  // no pivoting: L unit below the diagonal, U on and above it, in place
+  float W[NV][NV], rdiag[NV];
+  sfor<0, NV>([&]<int m>() { sfor<0, NV>([&]<int c>() { W[m][c] = (float)Ad[m][c]; }); });
+  sfor<0, NV>([&]<int p>() {
+    rdiag[p] = 1.0f / W[p][p];
+    sfor<p + 1, NV>([&]<int m>() {
+      W[m][p] = W[m][p] * rdiag[p];
+      sfor<p + 1, NV>([&]<int c>() { W[m][c] = fmaf(-W[m][p], W[p][c], W[m][c]); });
     });
   });
-  v4f blk[NB][NB];
-  sfor<0, NB>([&]<int I>() {
-    sfor<0, NB>([&]<int J>() {
-      sfor<0, 4>([&]<int i>() {
-        constexpr int r = 4 * I + i;
-        if constexpr (r < NV)
-          blk[I][J][i] = (float)Ad[J][r];
-        else
-          blk[I][J][i] = r == 4 * J + q ? 1.0f : 0.0f;
-      });
-    });
+  sfor<0, NV>([&]<int m>() {
+    x[m] = 0.0;
+    r[m] = bv[m];
   });
-  lu_factor<NB>(blk, q);
-  // the diagonal's reciprocals, to the quad
-  float rdiag[NV];
-  sfor<0, NV>([&]<int c>() { rdiag[c] = 1.0f / qb<c % 4>(blk[c / 4][c / 4][c % 4]); });
-  const double *bvp = a.y + 2 * NV * nc + at;
-  double bv[NB], x[NB], r[NB];
-  sfor<0, NB>([&]<int t>() {
-    const int m = 4 * t + q;
-    const double v = bvp[(m < NV ? m : 0) * nc];
-    bv[t] = real && m < NV ? v : 0.0;
-    x[t] = 0.0;
-    r[t] = bv[t];
-  });
-  // the flags are ints and a cell's count is set inside the loop: no lane mask lives out of it
-  int done = 0, count = a.maxsweeps + IM_FAIL;
-  int s = 0;
+  int count = a.maxsweeps + IM_FAIL;
 #pragma unroll 1
-  while (s < a.maxsweeps && !__all(done)) {
-    // z = (L U)^-1 r in FP32, replicated over the quad, in lu_solve's order
+  for (int s = 1; s <= a.maxsweeps; s++) {
     float z[NV];
-    sfor<0, NV>([&]<int m>() { z[m] = qb<m % 4>((float)r[m / 4]); });
-    sfor<1, NV>([&]<int m>() { sfor<0, m>([&]<int c>() { z[m] -= qb<c % 4>(blk[m / 4][c / 4][m % 4]) * z[c]; }); });
+    sfor<0, NV>([&]<int m>() {
+      z[m] = (float)r[m];
+      sfor<0, m>([&]<int c>() { z[m] -= W[m][c] * z[c]; });
+    });
     sfor<0, NV>([&]<int n>() {
       constexpr int m = NV - 1 - n;
-      sfor<m + 1, NV>([&]<int c>() { z[m] -= qb<c % 4>(blk[m / 4][c / 4][m % 4]) * z[c]; });
+      sfor<m + 1, NV>([&]<int c>() { z[m] -= W[m][c] * z[c]; });
       z[m] = z[m] * rdiag[m];
     });
-    // x += z on the lanes' own rows, for the cells still refining
-    sfor<0, NB>([&]<int t>() {
-      float zq = 0.0f;
-      sfor<0, 4>([&]<int p>() {
-        if constexpr (4 * t + p < NV) zq = q == p ? z[4 * t + p] : zq;
-      });
-      x[t] = done ? x[t] : x[t] + (double)zq;
-    });
-    // r = f - A x and the rows' scales, the products over the lane's columns summed over the quad
+    sfor<0, NV>([&]<int m>() { x[m] = x[m] + (double)z[m]; });
     int ok = 1;
     sfor<0, NV>([&]<int m>() {
-      double p = 0.0, sc = 0.0;
-      sfor<0, NB>([&]<int J>() {
-        const double ax = Ad[J][m] * x[J];
-        p = p + ax;
-        sc = sc + fabs(ax);
+      double p[4] = {0.0, 0.0, 0.0, 0.0}, sc[4] = {0.0, 0.0, 0.0, 0.0};
+      sfor<0, NV>([&]<int c>() {
+        const double ax = Ad[m][c] * x[c];
+        p[c % 4] = p[c % 4] + ax;
+        sc[c % 4] = sc[c % 4] + fabs(ax);
       });
-      p = qsum(p);
-      sc = qsum(sc);
-      if (q == m % 4) {
-        const double acc = bv[m / 4] - p, scale = fabs(bv[m / 4]) + sc;
-        r[m / 4] = done ? r[m / 4] : acc;
-        ok = ok & (fabs(acc) <= a.tol * scale ? 1 : 0);
-      }
+      r[m] = bv[m] - ((p[0] + p[1]) + (p[2] + p[3]));
+      const double scale = fabs(bv[m]) + ((sc[0] + sc[1]) + (sc[2] + sc[3]));
+      ok = ok & (fabs(r[m]) <= a.tol * scale ? 1 : 0);
     });
-    // the cell's rows are spread over its quad: done when all four lanes' rows are
-    ok = ok & __builtin_amdgcn_mov_dpp(ok, 0xB1, 0xf, 0xf, false);
-    ok = ok & __builtin_amdgcn_mov_dpp(ok, 0x4E, 0xf, 0xf, false);
-    s++;
-    count = !done && ok ? s : count;
-    done = done | ok;
+    if (ok) {
+      count = s;
+      break;
+    }
   }
-  if (!real) return;
-  if (q == 0) a.sweeps[cell] = a.first ? count : a.sweeps[cell] + count;
+  a.sweeps[cell] = a.first ? count : a.sweeps[cell] + count;
   const double h = *a.dt / a.parts;
-  sfor<0, NB>([&]<int t>() {
-    const int m = 4 * t + q;
-    if (m < NV) a.y[m * nc + cell] = a.y[m * nc + cell] + h * x[t];
-  });
+  sfor<0, NV>([&]<int m>() { a.y[m * nc + cell] = a.y[m * nc + cell] + h * x[m]; });
 }
 
 // the last part's end: the mean rate over the step, rho (Y_end - Y_start) / dt, into out as the
@@ -646,12 +596,10 @@ __global__ __launch_bounds__(FLAT) void k_iwhole(ImArgs a) {
   ijac_whole<M>(a, a.Q, i, j, k, im_code(a.b, i, j, k), (int)(g % 2));
 }
 
-// four waves of 16 cells per workgroup
-template <int NB, int NV>
-__global__ __launch_bounds__(256) void k_lusolve(ImArgs a) {
-  const int64_t grp = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (grp * IM_G >= a.ncell) return;
-  lu_refine_group<NB, NV>(a, grp, threadIdx.x & 63);
+template <int NV>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1))) void k_lusolve(ImArgs a) {
+  const int64_t cell = (int64_t)blockIdx.x * 64 + threadIdx.x;
+  if (cell < a.ncell) lu_refine_cell<NV>(a, cell);
 }
 
 template <class M>

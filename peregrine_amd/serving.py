@@ -5,7 +5,7 @@ Requests of three kinds arrive over time (a seeded Poisson stream in the benchma
 - ``Ignition``: a 0D H2-air reactor at constant volume (the reference's own ignition case,
   tests/chemint/cases.py:45-58, examples/autoIgnition.py:18-53), T0, p0 and the equivalence
   ratio phi given, integrated to ``tend`` by the implicit chemistry (linearly implicit Euler, the
-  per-cell systems factored in FP32 on the matrix cores and refined in FP64). Its result is the
+  per-cell systems factored in FP32 and refined in FP64). Its result is the
   final mass fractions and T and the time T took to rise by 400 K. Constant pressure is not built:
   the reference has no constant-pressure reactor either.
 - ``Tube``: Sod's shock tube on a walled line of n cells (the reference's walled lines,
