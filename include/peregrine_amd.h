@@ -262,6 +262,17 @@ int32_t pga_transport_grads(const pga_case *c, pga_view Q, pga_view state, pga_v
                             const pga_box *boxes, int32_t nboxes, pga_view Jinv, pga_view grads, pga_box gbox,
                             void *stream);
 
+/* pga_transport_grads with each boundary cell's gradients stored into the halos that mirror it too: up to
+ * 6 slabs of halo cells (as pga_halo places them: dst_start, src_start, extent, orient) of the
+ * gradients dst, whose source cells lie in gbox: what pga_copy_slabs would copy, with no copy. Not for a
+ * rotational periodic, whose gradients turn. nboxes 0 computes no transport. Replaces, with dqdxyz.mako,
+ * the exchange of peregrine/simulator/advecdiff/simulator.py:20-27. */
+int32_t pga_transport_grads_slabs(const pga_case *c, pga_view Q, pga_view state, pga_view trstate, pga_view hsp,
+                                  const pga_box *boxes, int32_t nboxes, pga_view Jinv, pga_view grads, pga_box gbox,
+                                  int32_t nslab, const pga_view *dst, const int32_t *dst_start,
+                                  const int32_t *src_start, const int32_t *extent, const int32_t *orient,
+                                  void *stream);
+
 /* The alpha-damped viscous flux of the faces of one axis in box (face indices), added to F:
  * Newtonian stress, Fourier heat, Fick species fluxes with the correction velocity, their
  * enthalpy flux and the stress work; xcc the cell centres, xf the face centres.

@@ -74,6 +74,7 @@ inline bool covers(const pga_view &v, const pga_box &b, int ncomp) {
 // is 1 2 3. As element offsets: base, the source cell s, and the step per destination axis.
 struct Placement {
   int64_t base, step[3];
+  pga_box src;  // the source cells
 };
 
 // false (with the error set) when orient is not three distinct axes or the source cells the box
@@ -103,6 +104,7 @@ inline bool placement(const char *who, const pga_view &src, const int32_t *s, co
     return false;
   }
   p.base = s[0] + s[1] * src.sj + s[2] * src.sk;
+  p.src = bs;
   return true;
 }
 

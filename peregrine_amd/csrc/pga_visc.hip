@@ -215,10 +215,28 @@ __global__ __launch_bounds__(256) void k_transport(const double *K, View Q, View
   transport_cell<NS, TRANS, EOS>(g, Q, st, Q.off(i, j, k), tr, hsp, tr.off(i, j, k), hsp.off(i, j, k), binary != 0);
 }
 
-// navstokes/kernels/dqdxyz.mako:16-41: the cell's gradients of u, v, w, T and the carried Y
+// The halo cells that mirror a box's cells: each slab a box of source cells, their copies' places in the
+// partner's gradients affine in the source cell's indexes. The gradients' launch stores a boundary cell's
+// gradients there too, what an exchange would copy: the exchange was a launch of its own that read every
+// component of the boundary back, 24 us for nine species at 80 x 48 x 56 and 9 for a Taylor-Green box of
+// 32^3, of a stage's 345 and 47. (The halo's gradients taken again from the partner's cells, along i a line
+// of memory for each value of the stencil, cost the gradients 16 us at 80 x 48 x 56.)
+struct GradSlab {
+  View gr;                      // the partner's gradients
+  Box3 src;                     // the cells it mirrors
+  int64_t base, st0, st1, st2;  // the copy of cell (i, j, k) at base + i st0 + j st1 + k st2
+};
+
+struct GradSlabs {
+  GradSlab s[6];
+  int n;
+};
+
+// navstokes/kernels/dqdxyz.mako:16-41: the cell's gradients of u, v, w, T and the carried Y, and their copies
+// in the halos that mirror it
 template <int NS>
-__device__ __forceinline__ void grads_cell(const View &Q, const View &st, const View &Jinv, const View &gr, int i, int j,
-                                           int k) {
+__device__ __forceinline__ void grads_cell(const View &Q, const View &st, const View &Jinv, const View &gr,
+                                           const GradSlabs &L, int i, int j, int k) {
 #pragma clang fp contract(off)
   constexpr int NGRAD = NS + 3;
   const int64_t o = Q.off(i, j, k);
@@ -230,7 +248,7 @@ __device__ __forceinline__ void grads_cell(const View &Q, const View &st, const 
     rm[a] = Q.at(o - d[a], 0);
     inv[a] = 1.0 / (rp[a] * rm[a]);
   }
-  const int64_t oj = Jinv.off(i, j, k), og = gr.off(i, j, k);
+  const int64_t oj = Jinv.off(i, j, k);
   double J[3][3];
 #pragma unroll
   for (int a = 0; a < 3; a++)
@@ -250,18 +268,28 @@ __device__ __forceinline__ void grads_cell(const View &Q, const View &st, const 
       }
     }
   }
+  const auto put = [&](const View &to, int64_t og) {
 #pragma unroll
-  for (int l = 0; l < NGRAD; l++)
+    for (int l = 0; l < NGRAD; l++)
 #pragma unroll
-    for (int e = 0; e < 3; e++)
-      gr.at(og, 3 * l + e) = dd[l][0] * J[0][e] + dd[l][1] * J[1][e] + dd[l][2] * J[2][e];
+      for (int e = 0; e < 3; e++)
+        to.at(og, 3 * l + e) = dd[l][0] * J[0][e] + dd[l][1] * J[1][e] + dd[l][2] * J[2][e];
+  };
+  put(gr, gr.off(i, j, k));
+#pragma unroll 1
+  for (int n = 0; n < L.n; n++) {
+    const GradSlab &s = L.s[n];
+    const unsigned a = i - s.src.s0, b = j - s.src.s1, c = k - s.src.s2;
+    if (a < (unsigned)s.src.e0 && b < (unsigned)s.src.e1 && c < (unsigned)s.src.e2)
+      put(s.gr, s.base + i * s.st0 + j * s.st1 + k * s.st2);
+  }
 }
 
 template <int NS>
-__global__ __launch_bounds__(256) void k_grads(View Q, View st, View Jinv, View gr, Box3 b) {
+__global__ __launch_bounds__(256) void k_grads(View Q, View st, View Jinv, View gr, GradSlabs L, Box3 b) {
   int i, j, k;
   if (!cell_of(b, i, j, k)) return;
-  grads_cell<NS>(Q, st, Jinv, gr, i, j, k);
+  grads_cell<NS>(Q, st, Jinv, gr, L, i, j, k);
 }
 
 // the transport over a box list and the gradients over a box in one launch: the transport's
@@ -269,7 +297,7 @@ __global__ __launch_bounds__(256) void k_grads(View Q, View st, View Jinv, View 
 template <int NS, int TRANS, int EOS>
 __global__ __launch_bounds__(256) void k_transport_grads(const double *K, View Q, View st, View tr, View hsp,
                                                          BoxList L, unsigned tblocks, int binary, View Jinv, View gr,
-                                                         Box3 gb) {
+                                                         Box3 gb, GradSlabs S) {
   int i, j, k;
   if (blockIdx.x < tblocks) {
     if (!boxlist_cell(L, blockIdx.x, i, j, k)) return;
@@ -278,7 +306,7 @@ __global__ __launch_bounds__(256) void k_transport_grads(const double *K, View Q
     return;
   }
   if (!flat_at(gb, blockIdx.x - tblocks, i, j, k)) return;
-  grads_cell<NS>(Q, st, Jinv, gr, i, j, k);
+  grads_cell<NS>(Q, st, Jinv, gr, S, i, j, k);
 }
 
 struct DiffArgs {
@@ -384,10 +412,57 @@ static int32_t grads_check(const char *who, const pga_case *c, pga_view Q, pga_v
   return PGA_OK;
 }
 
-extern "C" int32_t pga_transport_grads(const pga_case *c, pga_view Q, pga_view state, pga_view trstate, pga_view hsp,
-                                       const pga_box *boxes, int32_t nboxes, pga_view Jinv, pga_view grads,
-                                       pga_box gbox, void *stream) {
+// the halo slabs that mirror cells of gbox
+static int32_t grad_slabs(const char *who, const pga_case *c, pga_view Q, pga_box gbox, int32_t nslab,
+                          const pga_view *dst, const int32_t *dst_start, const int32_t *src_start,
+                          const int32_t *extent, const int32_t *orient, GradSlabs &L) {
+  L = GradSlabs{};
+  if (!nslab) return PGA_OK;
+  if (nslab < 0 || nslab > 6 || !dst || !dst_start || !src_start || !extent) {
+    set_error("%s: null argument or more than 6 slabs", who);
+    return PGA_EINVAL;
+  }
+  const int ncomp = 3 * (c->desc.ns + 3);
+  for (int n = 0; n < nslab; n++) {
+    const int32_t *ds = dst_start + 3 * n, *ss = src_start + 3 * n, *e = extent + 3 * n;
+    for (int m = 0; m < 3; m++)
+      PGA_REQUIRE(ds[m] >= 0 && ss[m] >= 0 && e[m] >= 0, "%s: slab %d has a negative start or extent", who, n);
+    if (!e[0] || !e[1] || !e[2]) continue;
+    PGA_REQUIRE(covers(dst[n], pga_box{{ds[0], ds[1], ds[2]}, {e[0], e[1], e[2]}}, ncomp),
+                "%s: slab %d reaches outside its gradients", who, n);
+    Placement pl;
+    if (!placement(who, Q, ss, orient ? orient + 3 * n : nullptr, e, 1, pl)) return PGA_ERANGE;
+    for (int m = 0; m < 3; m++)
+      PGA_REQUIRE(pl.src.start[m] >= gbox.start[m] &&
+                      pl.src.start[m] + pl.src.extent[m] <= gbox.start[m] + gbox.extent[m],
+                  "%s: slab %d mirrors cells outside the gradients' box", who, n);
+    GradSlab &s = L.s[L.n++];
+    s.gr = view(dst[n]), s.src = box3(pl.src);
+    // the slab's axis m runs along the source's axis A, forwards or back: inverted, a step of the source's
+    // A is one of the slab's m
+    const int64_t stride[3] = {1, dst[n].sj, dst[n].sk};
+    int64_t step[3] = {0, 0, 0};
+    s.base = 0;
+    for (int m = 0; m < 3; m++) {
+      const int code = orient ? orient[3 * n + m] : m + 1, A = (code - 1) % 3;
+      step[A] = code > 3 ? -stride[m] : stride[m];
+      s.base += ds[m] * stride[m] - step[A] * ss[A];
+    }
+    s.st0 = step[0], s.st1 = step[1], s.st2 = step[2];
+  }
+  return PGA_OK;
+}
+
+extern "C" int32_t pga_transport_grads_slabs(const pga_case *c, pga_view Q, pga_view state, pga_view trstate,
+                                             pga_view hsp, const pga_box *boxes, int32_t nboxes, pga_view Jinv,
+                                             pga_view grads, pga_box gbox, int32_t nslab, const pga_view *dst,
+                                             const int32_t *dst_start, const int32_t *src_start,
+                                             const int32_t *extent, const int32_t *orient, void *stream) {
   const char *who = "pga_transport_grads";
+  if (!c) {
+    set_error("%s: null case", who);
+    return PGA_EINVAL;
+  }
   if (!box_ok(gbox)) {
     set_error("%s: the gradients' box has a negative extent", who);
     return PGA_EINVAL;
@@ -396,6 +471,8 @@ extern "C" int32_t pga_transport_grads(const pga_case *c, pga_view Q, pga_view s
   int64_t total;
   int32_t rc = transport_list(who, c, Q, state, trstate, hsp, boxes, nboxes, L, total);
   if (rc != PGA_OK) return rc;
+  GradSlabs S;
+  if ((rc = grad_slabs(who, c, Q, gbox, nslab, dst, dst_start, src_start, extent, orient, S)) != PGA_OK) return rc;
   const bool grad = !empty(gbox);
   if (grad && (rc = grads_check(who, c, Q, state, Jinv, grads, gbox)) != PGA_OK) return rc;
   const int64_t gcells = grad ? (int64_t)gbox.extent[0] * gbox.extent[1] * gbox.extent[2] : 0;
@@ -407,24 +484,34 @@ extern "C" int32_t pga_transport_grads(const pga_case *c, pga_view Q, pga_view s
   const Box3 gb = grad ? box3(gbox) : Box3{};
   const dim3 grid(tblocks + gblocks);
   const bool done = dispatch_eos(d, [&]<int N, int E>() {
-    if (d.trans == TRANS_CONSTANT)
+    if (!tblocks)
+      hipLaunchKernelGGL((k_grads<N>), grid_of(gb), dim3(TI, TJ), 0, stream_of(stream), view(Q), view(state),
+                         view(Jinv), view(grads), S, gb);
+    else if (d.trans == TRANS_CONSTANT)
       hipLaunchKernelGGL((k_transport_grads<N, TRANS_CONSTANT, E>), grid, dim3(256), 0, stream_of(stream), c->K,
                          view(Q), view(state), view(trstate), view(hsp), L, tblocks, d.diffusion, view(Jinv),
-                         view(grads), gb);
+                         view(grads), gb, S);
     else if (d.trans == TRANS_KINETIC)
       hipLaunchKernelGGL((k_transport_grads<N, TRANS_KINETIC, E>), grid, dim3(256), 0, stream_of(stream), c->K,
                          view(Q), view(state), view(trstate), view(hsp), L, tblocks, d.diffusion, view(Jinv),
-                         view(grads), gb);
+                         view(grads), gb, S);
     else if constexpr (E == EOS_REAL)
       hipLaunchKernelGGL((k_transport_grads<N, TRANS_CHUNG, E>), grid, dim3(256), 0, stream_of(stream), c->K,
                          view(Q), view(state), view(trstate), view(hsp), L, tblocks, d.diffusion, view(Jinv),
-                         view(grads), gb);
+                         view(grads), gb, S);
   });
   if (!done) {
     set_error("%s: no kernel for %d species with eos %d", who, d.ns, d.eos);
     return PGA_EUNSUP;
   }
   return launched(who);
+}
+
+extern "C" int32_t pga_transport_grads(const pga_case *c, pga_view Q, pga_view state, pga_view trstate, pga_view hsp,
+                                       const pga_box *boxes, int32_t nboxes, pga_view Jinv, pga_view grads,
+                                       pga_box gbox, void *stream) {
+  return pga_transport_grads_slabs(c, Q, state, trstate, hsp, boxes, nboxes, Jinv, grads, gbox, 0, nullptr, nullptr,
+                                   nullptr, nullptr, nullptr, stream);
 }
 
 extern "C" int32_t pga_grads(const pga_case *c, pga_view Q, pga_view state, pga_view Jinv, pga_view grads,
@@ -442,7 +529,7 @@ extern "C" int32_t pga_grads(const pga_case *c, pga_view Q, pga_view state, pga_
 #define X(N)                                                                                                    \
   if (d.ns == N) {                                                                                              \
     hipLaunchKernelGGL((k_grads<N>), grid_of(b), dim3(TI, TJ), 0, stream_of(stream), view(Q), view(state),      \
-                       view(Jinv), view(grads), b);                                                             \
+                       view(Jinv), view(grads), GradSlabs{}, b);                                                \
     done = true;                                                                                                \
   }
   PGA_NS_CASES(X)

@@ -476,25 +476,38 @@ class Solver:
         self._exchange(lambda b: b.grads, 3 * self.sim.ngrad, 1, 0, 1)
 
     def transport_gradients(self, Q):
-        """transport() and gradients() for the fused step: a small block's two kernels in one launch
-        (pga_transport_grads, the same values), since it pays more for a launch than for its work; a
-        block of more than 2^16 cells in two (one launch holds the registers of the heavier kernel
-        for both: 0.8% slower per step on the 256 x 128 x 64 layer)."""
+        """transport() and gradients() for the fused step, a boundary cell's gradients stored into the halos
+        that mirror it, not exchanged (pga_transport_grads_slabs, the same values); a small block's
+        two kernels in one launch, since it pays more for a launch than for its work, a block of more
+        than 2^16 cells in two (one launch holds the registers of the heavier kernel for both: 0.8%
+        slower per step on the 256 x 128 x 64 layer). A rotational periodic's gradients turn: its case
+        exchanges them."""
+        turned = any(f.nbr is not None and f.rotperiodic for blk in self.blocks for f in blk.faces.values())
         for blk in self.blocks:
             boxes = [blk.interior_box()] + blk.halo_boxes(1)
             arr = (native.Box * len(boxes))(*boxes)
             Qv, st = blk.regs[Q].view(), blk.state.view()
+            head = (self.case.handle, Qv, st, blk.trstate.view(), blk.hsp.view(), arr)
+            tail = (blk.Jinv.view(), blk.grads.view(), blk.interior_box(), *self._gradient_slabs(blk, turned))
             if blk.ncells <= 1 << 16:
-                self._call("pga_transport_grads", self.case.handle, Qv, st, blk.trstate.view(), blk.hsp.view(), arr,
-                           len(boxes), blk.Jinv.view(), blk.grads.view(), blk.interior_box())
+                self._call("pga_transport_grads_slabs", *head, len(boxes), *tail)
             else:
-                self._call("pga_transport", self.case.handle, Qv, st, blk.trstate.view(), blk.hsp.view(), arr,
-                           len(boxes))
-                self._call("pga_grads", self.case.handle, Qv, st, blk.Jinv.view(), blk.grads.view(),
-                           blk.interior_box())
+                self._call("pga_transport", *head, len(boxes))
+                self._call("pga_transport_grads_slabs", *head, 0, *tail)
             for sponge in self.sponges:
                 self._call("pga_viscsponge", blk.xcc.view(), blk.trstate.view(), sponge.line, arr, len(boxes))
-        self._exchange(lambda b: b.grads, 3 * self.sim.ngrad, 1, 0, 1)
+        if turned:
+            self._exchange(lambda b: b.grads, 3 * self.sim.ngrad, 1, 0, 1)
+
+    def _gradient_slabs(self, blk, turned):
+        """The halo slabs that mirror a block's cells, as pga_transport_grads_slabs takes them."""
+        slabs = []
+        for dst in self.blocks if not turned else ():
+            slabs += [(dst.grads.view(), placement(dst, f, blk, 1)) for f in dst.faces.values()
+                      if f.nbr is not None and self.blocks[f.nbr] is blk]
+        n = len(slabs)
+        return (n, (native.View * n)(*[v for v, _ in slabs]),
+                *(native.ints([x for _, p in slabs for x in p[m]]) for m in range(4)))
 
     def fluxes(self, blk, Qv, st, slab=None, axes=(0, 1, 2), one_launch=False):
         """The advective flux of each axis, with the viscous flux added for a viscous case, then the
