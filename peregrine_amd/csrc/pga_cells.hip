@@ -132,7 +132,7 @@ __global__ __launch_bounds__(256) void k_production(const double *__restrict__ K
   double y[NS], w[NS];
 #pragma unroll
   for (int s = 0; s < NS; s++) y[s] = Y[(int64_t)s * n + p];
-  M::production(Gas<NS>{K}, C, rho[p], y, T[p], w);
+  M::production(Gas<NS>{K}, constants(C), rho[p], y, T[p], w);
 #pragma unroll
   for (int s = 0; s < NS; s++) omega[(int64_t)s * n + p] = w[s];
 }

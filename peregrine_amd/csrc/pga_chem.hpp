@@ -10,8 +10,8 @@ namespace pga {
 // g/(Ru T) of species n: its Gibbs polynomial in ln T plus h298/T (eos/kernels/species.mako:16-21),
 // Horner steps as explicit fused multiply-adds (the oracle evaluates the same sequence): the
 // polynomial's terms cancel by six orders, so the rounding sequence is fixed, not left to the compiler
-template <int NS, class P>
-__device__ __forceinline__ double gibbs_rt(const GasOf<NS, P> &g, int n, double logT, double Tinv) {
+template <int NS>
+__device__ __forceinline__ double gibbs_rt(const Gas<NS> &g, int n, double logT, double Tinv) {
 #pragma clang fp contract(off)
   double gr = 0.0;
 #pragma unroll
@@ -20,8 +20,8 @@ __device__ __forceinline__ double gibbs_rt(const GasOf<NS, P> &g, int n, double 
 }
 
 // cp/R and the internal energy of species n at T (eos/kernels/species.mako:3-27), u = ln T
-template <int NS, class P>
-__device__ __forceinline__ double cpR_species(const GasOf<NS, P> &g, int n, double u) {
+template <int NS>
+__device__ __forceinline__ double cpR_species(const Gas<NS> &g, int n, double u) {
 #pragma clang fp contract(off)
   double cpR = 0.0;
 #pragma unroll
@@ -29,8 +29,8 @@ __device__ __forceinline__ double cpR_species(const GasOf<NS, P> &g, int n, doub
   return cpR;
 }
 
-template <int NS, class P>
-__device__ __forceinline__ double e_species(const GasOf<NS, P> &g, int n, double T, double u, double Tinv) {
+template <int NS>
+__device__ __forceinline__ double e_species(const Gas<NS> &g, int n, double T, double u, double Tinv) {
 #pragma clang fp contract(off)
   double hRT = 0.0;
 #pragma unroll
@@ -65,7 +65,7 @@ __device__ __forceinline__ void cell_source(const Gas<M::NS> &g, const double *_
   const double rho = Q.at(o, 0), rhoinv = 1.0 / rho;
   double Y[NS], omega[NS];
   massfrac<NS>(Q, o, rhoinv, Y);
-  M::production(g, C, rho, Y, st.at(o, 1), omega);
+  M::production(g, constants(C), rho, Y, st.at(o, 1), omega);
 #pragma unroll
   for (int l = 0; l < 5; l++) dQ.at(o, l) = 0.0;
 #pragma unroll

@@ -78,12 +78,21 @@ __host__ __device__ constexpr Offsets offsets(int ns) {
   return o;
 }
 
-// the species constants of a case with NS species, read at compile-time offsets from a
-// wave-uniform pointer: the compiler turns each read into a scalar load
-template <int NS, class P>
-struct GasOf {
+// A constant table in the constant address space: its reads are scalar loads wherever they stand. Through a
+// plain pointer they are vector loads, a register pair and a wait each, behind a store the compiler cannot
+// tell apart (the transport's, between mu and the species' values; the EOS's in a launch that stores Q before
+// it; another branch's): the transport of nine species by binary pairs went from 83 to 56 us at 80 x 48 x 56,
+// the sub-stepped 50 x 37 x 45 step from 315 to 278 us, the reacting 128^3 block's faces from 371 to 358 us.
+using Constants = const __attribute__((address_space(4))) double *;
+__device__ __forceinline__ Constants constants(const double *p) { return (Constants)(uintptr_t)p; }
+
+// the species constants of a case with NS species, read at compile-time offsets
+template <int NS>
+struct Gas {
   static constexpr Offsets O = offsets(NS);
-  P K;
+  Constants K;
+  __device__ __forceinline__ explicit Gas(Constants k) : K(k) {}
+  __device__ __forceinline__ explicit Gas(const double *k) : K(constants(k)) {}
   __device__ __forceinline__ double MW(int n) const { return K[O.MW + n]; }
   __device__ __forceinline__ double MWinv(int n) const { return K[O.MWinv + n]; }
   __device__ __forceinline__ double Rsp(int n) const { return K[O.Rsp + n]; }
@@ -125,14 +134,6 @@ struct GasOf {
   __device__ __forceinline__ double bathof(int n, int k) const { return K[O.bathof + n * NS + k]; }
   __device__ __forceinline__ double diffmeta(int i) const { return K[O.diffmeta + i]; }
 };
-
-template <int NS>
-using Gas = GasOf<NS, const double *__restrict__>;
-
-// a constant table in the constant address space: its reads are scalar loads wherever they stand, where
-// through a plain pointer they are vector loads, a register pair each, behind a store of another branch
-using Constants = const __attribute__((address_space(4))) double *;
-__device__ __forceinline__ Constants constants(const double *p) { return (Constants)(uintptr_t)p; }
 
 // ---------------------------------------------------------------------------
 // views and launch shapes

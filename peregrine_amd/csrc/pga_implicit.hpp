@@ -191,8 +191,8 @@ __device__ __forceinline__ void rhs0d(const Gas<M::NS> &g, const double *__restr
   for (int n = 0; n < NS; n++) Y[n] = y[n];
   const double T = y[NS];
   typename M::Rates s;
-  M::ratestate(g, C, rho, Y, T, s);
-  M::template fold<false>(C, s, rate, D);
+  M::ratestate(g, constants(C), rho, Y, T, s);
+  M::template fold<false>(constants(C), s, rate, D);
   double cv = 0.0, dTdt = 0.0;
 #pragma unroll
   for (int n = 0; n < NS; n++) {
@@ -341,7 +341,7 @@ __device__ __forceinline__ void ijac_part(const ImArgs &a, double T, double *lds
 #pragma clang fp contract(off)
   constexpr int NS = M::NS, NT = sizeof(typename M::TCache) / sizeof(double);
   const ImGroup X(a, lds);
-  const GasOf<NS, Constants> g{X.K};
+  const Gas<NS> g{X.K};
   const auto put = [&](int e, double v) { X(e) = v; };
   M::template tstate_part<G>(g, X.C, T, put);
   const double logT = tlog(T), Tinv = 1.0 / T;

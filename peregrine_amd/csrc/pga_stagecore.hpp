@@ -240,7 +240,7 @@ __device__ __forceinline__ void rates_cell(const double *__restrict__ K, const d
   const double rho = Q.at(o, 0), rhoinv = 1.0 / rho;
   double Y[NS], omega[NS];
   massfrac<NS>(Q, o, rhoinv, Y);
-  M::production(Gas<NS>{K}, C, rho, Y, st.at(o, 1), omega);
+  M::production(Gas<NS>{K}, constants(C), rho, Y, st.at(o, 1), omega);
   const int64_t orr = rates.off(i, j, k);
 #pragma unroll
   for (int n = 0; n < NS - 1; n++) rates.at(orr, n) = omega[n];

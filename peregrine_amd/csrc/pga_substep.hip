@@ -45,12 +45,12 @@ __device__ int integrate(const Gas<M::NS> &g, const double *__restrict__ C, int 
 #pragma unroll 1
   for (; sub < limit && remaining > SUB_STEPFRAC; sub++) {
     typename M::Rates s;
-    M::ratestate(g, C, rho, Y, T, s);
+    M::ratestate(g, constants(C), rho, Y, T, s);
     // the first substep's fold carries the destruction rates the exit relaxes by
     if (EXIT && sub == 0)
-      M::template fold<true>(C, s, rate, D);
+      M::template fold<true>(constants(C), s, rate, D);
     else
-      M::template fold<false>(C, s, rate, D);
+      M::template fold<false>(constants(C), s, rate, D);
     // the limiting species by cross-multiplying, one quotient at the end; a trace species counts
     double abest = 0.0, bbest = 0.0;
 #pragma unroll

@@ -135,7 +135,7 @@ def render(name, records, sets, ns):
     if sets:
         w(f"    double ctb[{len(sets)}], logtb[{len(sets)}];")
     w("  };")
-    w("  __device__ __forceinline__ static void ratestate(const Gas<NS> &g, const double *__restrict__ C, double rho,")
+    w("  __device__ __forceinline__ static void ratestate(const Gas<NS> &g, Constants C, double rho,")
     w("                                                   const double (&Y)[NS], double T, Rates &s) {")
     w("#pragma clang fp contract(off)")
     w("    s.logT = tlog(T);")
@@ -163,7 +163,7 @@ def render(name, records, sets, ns):
     w("  }")
     # the fold, finiterate.mako:185-236: omega and, with WITHD, the destruction rates D
     w("  template <bool WITHD>")
-    w("  __device__ __forceinline__ static void fold(const double *__restrict__ C, const Rates &s, double (&omega)[NS],")
+    w("  __device__ __forceinline__ static void fold(Constants C, const Rates &s, double (&omega)[NS],")
     w("                                              double (&D)[NS]) {")
     _fold_prologue(w, L, records, ns, logform, product)
     _fold_reactions(w, L, records)
@@ -192,7 +192,7 @@ def render(name, records, sets, ns):
     off["kx"] = at + ns
     _tstate_part(w, L, records, ns, off, logform, product)
     _fold_columns(w, L, records, sets, ns, off, logform, product)
-    w("  __device__ __forceinline__ static void production(const Gas<NS> &g, const double *__restrict__ C,")
+    w("  __device__ __forceinline__ static void production(const Gas<NS> &g, Constants C,")
     w("                                                    double rho, const double (&Y)[NS], double T, double (&omega)[NS]) {")
     w("    Rates s;")
     w("    ratestate(g, C, rho, Y, T, s);")
@@ -396,8 +396,8 @@ def _tstate_part(w, L, records, ns, off, logform, product):
     """One of GROUPS shares of the TCache at T, each value put (put(index, value)) where TCache's member lies."""
     groups = -(-ns // COLUMNS)
     w(f"  static constexpr int COLS = {COLUMNS}, GROUPS = {groups};")
-    w("  template <int G, class GA, class PUT>")
-    w("  __device__ __forceinline__ static void tstate_part(const GA &g, Constants C, double T, const PUT &put) {")
+    w("  template <int G, class PUT>")
+    w("  __device__ __forceinline__ static void tstate_part(const Gas<NS> &g, Constants C, double T, const PUT &put) {")
     w("#pragma clang fp contract(off)")
     w("    const double logT = tlog(T), Tinv = 1.0 / T;")
     w(f"    double gRT[{ns}];")
