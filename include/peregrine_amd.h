@@ -229,6 +229,13 @@ int32_t pga_halo(const pga_case *c, int32_t ntask, const pga_view *Qdst, const p
                  const int32_t *dst_start, const int32_t *src_start, const int32_t *extent, const int32_t *orient,
                  const double *rot, pga_view stdst, pga_view stguess, void *stream);
 
+/* pga_halo and pga_rates over box in one launch, the same values as the two calls: the halo pass writes halo
+ * cells, the rates read the cells of box, which holds none of them. The kernels replaced are those calls'. */
+int32_t pga_halo_rates(const pga_case *c, int32_t ntask, const pga_view *Qdst, const pga_view *Qsrc,
+                       const int32_t *dst_start, const int32_t *src_start, const int32_t *extent,
+                       const int32_t *orient, const double *rot, pga_view stdst, pga_view stguess, pga_view Q,
+                       pga_view state, pga_view rates, pga_box box, void *stream);
+
 /* --- the viscous terms (Navier-Stokes) ---------------------------------------------------- */
 
 /* Per cell of up to 8 boxes: trstate = [mu, kappa, D_0 .. D_{ns-1}] by the case's transport model

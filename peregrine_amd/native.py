@@ -105,6 +105,8 @@ SIGNATURES = {
     "pga_rates": (_i32, [C.c_void_p, View, View, View, Box, C.c_void_p]),
     "pga_halo": (_i32, [C.c_void_p, _i32, C.POINTER(View), C.POINTER(View), _ip, _ip, _ip, _ip, _dp, View, View,
                         C.c_void_p]),
+    "pga_halo_rates": (_i32, [C.c_void_p, _i32, C.POINTER(View), C.POINTER(View), _ip, _ip, _ip, _ip, _dp, View, View,
+                              View, View, View, Box, C.c_void_p]),
     "pga_transport": (_i32, [C.c_void_p, View, View, View, View, C.POINTER(Box), _i32, C.c_void_p]),
     "pga_grads": (_i32, [C.c_void_p, View, View, View, View, Box, C.c_void_p]),
     "pga_transport_grads": (_i32, [C.c_void_p, View, View, View, View, C.POINTER(Box), _i32, View, View, Box,

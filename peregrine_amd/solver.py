@@ -678,8 +678,9 @@ class Solver:
         self.advance(n)
 
     # -- the fused stage ------------------------------------------------------
-    def _halo_pass(self, qin):
-        """Each block's halo slabs from its partners' interior planes, and the EOS over them."""
+    def _halo_pass(self, qin, rates=False):
+        """Each block's halo slabs from its partners' interior planes, and the EOS over them; rates: and its
+        interior's coupled production rates, which need no halo, in the same launch."""
         for blk in self.blocks:
             dsts, srcs, ds, ss, es, os, rots = [], [], [], [], [], [], []
             for f in blk.faces.values():
@@ -696,9 +697,13 @@ class Solver:
                 rots += list(f.rot.ravel()) if f.rotperiodic else [1.0, 0, 0, 0, 1.0, 0, 0, 0, 1.0]
             n = len(dsts)
             turns = native.dbls(rots) if any(f.rotperiodic for f in blk.faces.values() if f.nbr is not None) else None
-            self._call("pga_halo", self.case.handle, n, (native.View * n)(*dsts), (native.View * n)(*srcs),
-                       native.ints(ds), native.ints(ss), native.ints(es), native.ints(os), turns, blk.state.view(),
-                       blk.state.view())
+            st = blk.state.view()
+            args = (self.case.handle, n, (native.View * n)(*dsts), (native.View * n)(*srcs), native.ints(ds),
+                    native.ints(ss), native.ints(es), native.ints(os), turns, st, st)
+            if rates:
+                self._call("pga_halo_rates", *args, blk.regs[qin].view(), st, blk.rates.view(), blk.interior_box())
+            else:
+                self._call("pga_halo", *args)
 
     def _combine_terms(self, n):
         """The stage's combine as (source, weight, times dt) terms in the reference's order: its
@@ -875,8 +880,10 @@ class Solver:
         divergence + source + combine + EOS, in place on the reference's stage registers."""
         kc = int(self.cfg["backend-mi355x"]["k-chunk"])
         for n, regs in enumerate(self.integ.stageregs(self.regs)):
+            mixed = False
             if regs.Q not in self.readied:
-                self._halo_pass(regs.Q)
+                mixed = self.sim.chemistry and self.sim.chemkind == "coupled"
+                self._halo_pass(regs.Q, rates=mixed)
                 self.wall_halos(regs.Q)
                 if self.sim.viscous:
                     self.transport_gradients(regs.Q)
@@ -898,7 +905,7 @@ class Solver:
                 with stream:
                     box = blk.interior_box()
                     Qin, st = blk.regs[regs.Q].view(), blk.state.view()
-                    if self.sim.chemistry:
+                    if self.sim.chemistry and not mixed:
                         self.chemistry_source(blk, Qin, blk.rates.view(), False)
                     rates = blk.rates.view() if self.sim.chemistry else native.View()
                     march = self._march(blk, regs, first)
