@@ -22,40 +22,46 @@
 
 namespace pga {
 
-// the divergence, the source and the RK combine of a column of cells: memory-bound
+// the divergence, the source and the RK combine of a column of cells: memory-bound. blockIdx.z: the row group,
+// then the planes
 template <int NE, bool CHEM>
 __global__ __launch_bounds__(WT) void k_stage(StageArgs a) {
   const int i = a.s0 + blockIdx.x * WI + (threadIdx.x & (WI - 1));
   const int j = a.s1 + blockIdx.y * WJ + threadIdx.x / WI;
   if (i >= a.s0 + a.n0 || j >= a.s1 + a.n1) return;
-  const int kbeg = a.s2 + blockIdx.z * a.kc;
-  stage_cells<NE, CHEM>(a, i, j, kbeg, min(kbeg + a.kc, a.s2 + a.n2));
+  const int kz = blockIdx.z / a.groups, lbeg = (blockIdx.z - kz * a.groups) * a.rows, kbeg = a.s2 + kz * a.kc;
+  stage_cells<NE, CHEM>(a, i, j, kbeg, min(kbeg + a.kc, a.s2 + a.n2), lbeg, min(lbeg + a.rows, NE));
 }
 
-// a small block's stage and the EOS of its result in one launch: each thread's cells after its
-// column's combine (a block of a few thousand cells is bound by launches, not by the registers the
-// two phases hold at once, which at 128^3 favour the two launches apart)
+// The row groups a block's stage goes in. A thread waits on memory once a row: a block too small to fill the
+// SIMDs waits for its rows one after another, so below 2^17 cells (two waves to each of the 1024 SIMDs) it takes
+// them by several threads, as many as bring eight waves to each (the rows need nothing of each other but 1/J).
+// Nine species: 25 to 20 us a launch at 61 x 47 x 33, the 50 x 37 x 45
+// sub-stepped step from 278 to 260; the 215 040 cells of 80 x 48 x 56 take 41.8 us whole and 44.2 in three groups
+static void row_groups(StageArgs &a, int ne) {
+  const int64_t cells = std::max<int64_t>(1, (int64_t)a.n0 * a.n1 * a.n2);
+  const int64_t want = cells > (int64_t(1) << 17) ? 1 : std::min<int64_t>(ne, (int64_t(8) * 1024 * 64 + cells - 1) / cells);
+  a.rows = (ne + (int)want - 1) / (int)want;
+  a.groups = (ne + a.rows - 1) / a.rows;
+}
+
+// a small block's stage and the EOS of its result in one launch, for a few rows: each cell's reads at once, its
+// EOS from the new Q in registers (a block of a few thousand cells is bound by launches and waits)
 template <int NS, int EOS, bool CHEM>
 __global__ __launch_bounds__(WT) void k_stage_whole(StageArgs a) {
   const int i = a.s0 + blockIdx.x * WI + (threadIdx.x & (WI - 1));
   const int j = a.s1 + blockIdx.y * WJ + threadIdx.x / WI;
   if (i >= a.s0 + a.n0 || j >= a.s1 + a.n1) return;
   const int kbeg = a.s2 + blockIdx.z * a.kc, kend = min(kbeg + a.kc, a.s2 + a.n2);
-  if constexpr (NS + 4 <= 8) {
-    // a few rows: each cell's reads at once, its EOS from the new Q in registers
-    const Gas<NS> g{a.K};
-    const double dt = *a.dt;
-    for (int k = kbeg; k < kend; k++) {
-      const double Tguess = a.stin.at(a.stin.off(i, j, k), 1);
-      double Qn[NS + 4];
-      stage_cell_regs<NS + 4, CHEM>(a, i, j, k, dt, Qn);
-      EosState s;
-      fromQ_regs<NS, EOS>(g, Qn, Tguess, s);
-      store_state<EOS>(a.stout, a.stout.off(i, j, k), s);
-    }
-  } else {
-    stage_cells<NS + 4, CHEM>(a, i, j, kbeg, kend);
-    for (int k = kbeg; k < kend; k++) eos_cell<NS, EOS>(a.K, a.Qout, a.stin, a.stout, i, j, k);
+  const Gas<NS> g{a.K};
+  const double dt = *a.dt;
+  for (int k = kbeg; k < kend; k++) {
+    const double Tguess = a.stin.at(a.stin.off(i, j, k), 1);
+    double Qn[NS + 4];
+    stage_cell_regs<NS + 4, CHEM>(a, i, j, k, dt, Qn);
+    EosState s;
+    fromQ_regs<NS, EOS>(g, Qn, Tguess, s);
+    store_state<EOS>(a.stout, a.stout.off(i, j, k), s);
   }
 }
 
@@ -205,20 +211,24 @@ static int32_t stage_impl(const char *who, const pga_case *c, pga_view Qin, pga_
   a.kc = kchunk;
   const dim3 grid((a.n0 + WI - 1) / WI, (a.n1 + WJ - 1) / WJ, (a.n2 + kchunk - 1) / kchunk);
   const Box3 b = box3(box);
-  // a block of at most 2^16 cells (up to 40^3) in one launch, a larger one in two
+  // a block of at most 2^16 cells (up to 40^3) whose rows fit registers in one launch, any other in two
   const bool whole = (int64_t)a.n0 * a.n1 * a.n2 <= (int64_t(1) << 16);
+  row_groups(a, ne);
+  const dim3 rgrid(grid.x, grid.y, grid.z * a.groups);
   const bool done = dispatch_eos(d, [&]<int N, int E>() {
-    if (whole) {
-      if (chem)
-        hipLaunchKernelGGL((k_stage_whole<N, E, true>), grid, dim3(WT), 0, stream_of(stream), a);
-      else
-        hipLaunchKernelGGL((k_stage_whole<N, E, false>), grid, dim3(WT), 0, stream_of(stream), a);
-      return;
+    if constexpr (N + 4 <= 8) {
+      if (whole) {
+        if (chem)
+          hipLaunchKernelGGL((k_stage_whole<N, E, true>), grid, dim3(WT), 0, stream_of(stream), a);
+        else
+          hipLaunchKernelGGL((k_stage_whole<N, E, false>), grid, dim3(WT), 0, stream_of(stream), a);
+        return;
+      }
     }
     if (chem)
-      hipLaunchKernelGGL((k_stage<N + 4, true>), grid, dim3(WT), 0, stream_of(stream), a);
+      hipLaunchKernelGGL((k_stage<N + 4, true>), rgrid, dim3(WT), 0, stream_of(stream), a);
     else
-      hipLaunchKernelGGL((k_stage<N + 4, false>), grid, dim3(WT), 0, stream_of(stream), a);
+      hipLaunchKernelGGL((k_stage<N + 4, false>), rgrid, dim3(WT), 0, stream_of(stream), a);
     hipLaunchKernelGGL((k_stage_eos<N, E>), grid_of(b), dim3(TI, TJ), 0, stream_of(stream), c->K, a.Qout, a.stin,
                        a.stout, b);
   });

@@ -35,6 +35,7 @@ struct StageArgs {
   const double *dt;
   int s0, s1, s2, n0, n1, n2;
   int kc;
+  int groups, rows;  // the conserved rows in groups of so many, a thread a cell and group
   int q0;  // whether a combine term reads Q0 (RK3's first stage reads only Qin and dQ)
 };
 
@@ -157,11 +158,12 @@ __device__ __forceinline__ void stage_cell_regs(const StageArgs &a, int i, int j
   }
 }
 
-// The divergence, the source and the RK combine of the cells (i, j, kbeg..kend-1) of one column:
-// memory-bound. A row at a time in a rolled loop keeps ~30 registers, so eight waves per SIMD hide
+// The divergence, the source and the RK combine of rows lbeg..lend-1 of the cells (i, j, kbeg..kend-1) of one
+// column: memory-bound. A row at a time in a rolled loop keeps ~30 registers, so eight waves per SIMD hide
 // the loads' latency
 template <int NE, bool CHEM>
-__device__ __forceinline__ void stage_cells(const StageArgs &a, int i, int j, int kbeg, int kend) {
+__device__ __forceinline__ void stage_cells(const StageArgs &a, int i, int j, int kbeg, int kend, int lbeg = 0,
+                                            int lend = NE) {
   const View &kF = a.kF;
   const double dt = *a.dt;
 #pragma unroll 1
@@ -172,7 +174,7 @@ __device__ __forceinline__ void stage_cells(const StageArgs &a, int i, int j, in
     const int64_t orr = CHEM ? a.rates.off(i, j, k) : 0;
     const double J = __builtin_nontemporal_load(&a.det.at(a.det.off(i, j, k), 0));
 #pragma unroll 1
-    for (int l = 0; l < NE; l++)
+    for (int l = lbeg; l < lend; l++)
       stage_row<CHEM>(a, l, kF.at(fkl, l), kF.at(fkh, l), o, o0, oo, fil, fjl, orr, J, dt, i, j, k);
   }
 }
