@@ -210,26 +210,23 @@ __global__ __launch_bounds__(FLAT) void kb_iwhole(BArgs a, ImArgs im) {
   ijac_whole<M>(im, B.Q[a.q], i, j, k, g * FLAT + threadIdx.x, (int)(gs % 2));
 }
 
-// the places of a tile's overhang (no cell): the identity and a zero right-hand side, once a call,
-// so the quad-per-cell solve finds every place of its groups defined and settles them in one sweep
+// the part's solve, 64 of a tile's places a workgroup, as k_lusolve; the places of a tile's overhang hold no
+// cell and count one sweep
 template <int NV>
-__global__ __launch_bounds__(FLAT) void kb_ivoid(BArgs a, ImArgs im) {
-  const int64_t g = xcd_block();
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1))) void kb_lusolve(BArgs a, ImArgs im) {
+  constexpr int64_t S = FLAT / 64;
+  const int64_t gs = blockIdx.x, g = gs / S;
   const int n = bfind(a.prefix, a.nblocks, g);
   const BBlock &B = a.blocks[n];
+  const unsigned at = (unsigned)(gs - g * S) * 64 + threadIdx.x;
+  const int64_t code = g * FLAT + at;
   int i, j, k;
-  if (flat_at(B.b, g - a.prefix[n], i, j, k)) return;
-  for (int m = 0; m <= NV; m++) ijac_void<NV>(im, g * FLAT + threadIdx.x, m);
-}
-
-template <class M>
-__global__ __launch_bounds__(FLAT) void kb_iend(BArgs a, ImArgs im) {
-  const int64_t g = xcd_block();
-  const int n = bfind(a.prefix, a.nblocks, g);
-  const BBlock &B = a.blocks[n];
-  int i, j, k;
-  if (!flat_at(B.b, g - a.prefix[n], i, j, k)) return;
-  iend_cell<M>(im, B.Q[a.q], B.rates, i, j, k, g * FLAT + threadIdx.x);
+  if (!cell_at(B.b, (unsigned)(g - a.prefix[n]) * FLAT + at, i, j, k)) {
+    im.sweeps[code] = im.first ? 1 : im.sweeps[code] + 1;
+    return;
+  }
+  const View Q = B.Q[a.q], out = B.rates;
+  lu_refine_cell<NV>(im, Q, out, i, j, k, code);
 }
 
 // the tiles of each kind a block takes
@@ -593,15 +590,13 @@ extern "C" int32_t pga_batch_implicit(const pga_batch *h, const pga_implicit_opt
 #define X(NAME, IDX)                                                                             \
   if (d.mechanism == IDX) {                                                                      \
     constexpr int NV = Mech_##NAME::NS + 1;                                                      \
-    hipLaunchKernelGGL((kb_ivoid<NV>), grid, dim3(FLAT), 0, s, a, im);                           \
     for (int part = 0; part < o->parts; part++) {                                                \
       im.first = part == 0, im.last = part == o->parts - 1;                                      \
       hipLaunchKernelGGL((kb_icol<Mech_##NAME>), dim3(grid.x * (FLAT / IM_CELLS)),               \
                          dim3(Mech_##NAME::GROUPS * IM_CELLS), im_cols_lds<Mech_##NAME>, s, a, im); \
       hipLaunchKernelGGL((kb_iwhole<Mech_##NAME>), dim3(grid.x * 2), dim3(FLAT), 0, s, a, im);   \
-      hipLaunchKernelGGL((k_lusolve<NV>), dim3((unsigned)((cells + 63) / 64)), dim3(64), 0, s, im); \
+      hipLaunchKernelGGL((kb_lusolve<NV>), dim3((unsigned)(cells / 64)), dim3(64), 0, s, a, im); \
     }                                                                                            \
-    hipLaunchKernelGGL((kb_iend<Mech_##NAME>), grid, dim3(FLAT), 0, s, a, im);                  \
     done = true;                                                                                 \
   }
   PGA_MECHANISMS(X)

@@ -105,7 +105,6 @@ extern "C" int32_t pga_implicit(const pga_case *c, const pga_implicit_opts *o, p
       hipLaunchKernelGGL((k_iwhole<Mech_##NAME>), dim3(grid.x * 2), dim3(FLAT), 0, s, a);        \
       hipLaunchKernelGGL((k_lusolve<NV>), dim3((unsigned)((cells + 63) / 64)), dim3(64), 0, s, a); \
     }                                                                                             \
-    hipLaunchKernelGGL((k_iend<Mech_##NAME>), grid, dim3(FLAT), 0, s, a);                        \
     done = true;                                                                                  \
   }
   PGA_MECHANISMS(X)

@@ -468,20 +468,6 @@ __device__ __forceinline__ void ijac_whole(const ImArgs &a, const View &Q, int i
   for (int r = 0; r < NV; r++) a.A[a64_at<NV>(code, r, NS)] = (r == NS ? 1.0 : 0.0) - (f1[r] - fh[r * nc]) * hd;
 }
 
-// what a slice of the columns' launch leaves for a work place that holds no cell (a tile's overhang in
-// a table of blocks): the identity's column, or a zero right-hand side, which the solve takes in one
-// sweep
-template <int NV>
-__device__ __forceinline__ void ijac_void(const ImArgs &a, int64_t code, int m) {
-  if (m < NV) {
-#pragma unroll
-    for (int r = 0; r < NV; r++) a.A[a64_at<NV>(code, r, m)] = r == m ? 1.0 : 0.0;
-  } else {
-#pragma unroll
-    for (int r = 0; r < NV; r++) a.y[2 * NV * a.ncell + r * a.ncell + code] = 0.0;
-  }
-}
-
 // The part's solve and step, a lane per cell: (I - h J) x = f(y) by iterative refinement, then y += h x. The
 // lane loads its FP64 matrix once and keeps it, and the FP32 factors of its rounding, in registers, at one
 // wave a SIMD; each sweep solves L U z = r in FP32, adds z to x and takes r = f - A x in FP64 with the row
@@ -495,9 +481,15 @@ __device__ __forceinline__ void ijac_void(const ImArgs &a, int64_t code, int m) 
 // matrices would be three passes over HBM.
 //
 // The sums go column c into the (c mod 4)-th of four partial sums, then ((0) + (1)) + ((2) + (3)).
+//
+// The last part's end, the mean rate over the step, rho (Y_end - Y_start) / dt, goes from the lane's x into
+// out as the sub-stepped form begins dQ (or into the rates): a launch of its own read y and Q again, 11 us
+// for 64^3 cells.
 template <int NV>
-__device__ __forceinline__ void lu_refine_cell(const ImArgs &a, int64_t cell) {
+__device__ __forceinline__ void lu_refine_cell(const ImArgs &a, const View &Q, const View &out, int i, int j, int k,
+                                               int64_t cell) {
 #pragma clang fp contract(off)
+  constexpr int NS = NV - 1;
   const int64_t nc = a.ncell;
   const double *A = a.A + a64_at<NV>(cell, 0, 0), *bvp = a.y + 2 * NV * nc + cell;
   double Ad[NV][NV], bv[NV], x[NV], r[NV];
@@ -550,32 +542,23 @@ __device__ __forceinline__ void lu_refine_cell(const ImArgs &a, int64_t cell) {
   }
   a.sweeps[cell] = a.first ? count : a.sweeps[cell] + count;
   const double h = *a.dt / a.parts;
-  sfor<0, NV>([&]<int m>() { a.y[m * nc + cell] = a.y[m * nc + cell] + h * x[m]; });
-}
-
-// the last part's end: the mean rate over the step, rho (Y_end - Y_start) / dt, into out as the
-// sub-stepped form begins dQ (or into the rates)
-template <class M>
-__device__ __forceinline__ void iend_cell(const ImArgs &a, const View &Q, const View &out, int i, int j, int k,
-                                          int64_t code) {
-#pragma clang fp contract(off)
-  constexpr int NS = M::NS;
-  const int64_t nc = a.ncell;
-  const int64_t o = Q.off(i, j, k);
+  sfor<0, NV>([&]<int m>() { x[m] = a.y[m * nc + cell] + h * x[m]; });
+  if (!a.last) {
+    sfor<0, NV>([&]<int m>() { a.y[m * nc + cell] = x[m]; });
+    return;
+  }
+  const int64_t o = Q.off(i, j, k), oo = out.off(i, j, k);
   const double rho = Q.at(o, 0), rhoinv = 1.0 / rho;
   double Ys[NS];
   massfrac<NS>(Q, o, rhoinv, Ys);
   const double rdt = rho / *a.dt;
-  const int64_t oo = out.off(i, j, k);
+  const int row = a.begin_dQ ? 5 : 0;
   if (a.begin_dQ) {
 #pragma unroll
     for (int l = 0; l < 5; l++) out.at(oo, l) = 0.0;
-#pragma unroll
-    for (int n = 0; n < NS - 1; n++) out.at(oo, 5 + n) = (a.y[n * nc + code] - Ys[n]) * rdt;
-  } else {
-#pragma unroll
-    for (int n = 0; n < NS - 1; n++) out.at(oo, n) = (a.y[n * nc + code] - Ys[n]) * rdt;
   }
+#pragma unroll
+  for (int n = 0; n < NS - 1; n++) out.at(oo, row + n) = (x[n] - Ys[n]) * rdt;
 }
 
 template <class M>
@@ -598,15 +581,9 @@ __global__ __launch_bounds__(FLAT) void k_iwhole(ImArgs a) {
 
 template <int NV>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1))) void k_lusolve(ImArgs a) {
-  const int64_t cell = (int64_t)blockIdx.x * 64 + threadIdx.x;
-  if (cell < a.ncell) lu_refine_cell<NV>(a, cell);
-}
-
-template <class M>
-__global__ __launch_bounds__(FLAT) void k_iend(ImArgs a) {
+  const unsigned cell = blockIdx.x * 64 + threadIdx.x;
   int i, j, k;
-  if (!flat_cell_of(a.b, i, j, k)) return;
-  iend_cell<M>(a, a.Q, a.out, i, j, k, im_code(a.b, i, j, k));
+  if (cell < (unsigned)a.ncell && cell_at(a.b, cell, i, j, k)) lu_refine_cell<NV>(a, a.Q, a.out, i, j, k, cell);
 }
 
 }  // namespace pga
