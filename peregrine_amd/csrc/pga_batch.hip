@@ -587,18 +587,24 @@ extern "C" int32_t pga_batch_implicit(const pga_batch *h, const pga_implicit_opt
   const dim3 grid = tiles_grid(h->total[BK_CELLS]);
   hipStream_t s = stream_of(stream);
   bool done = false;
-#define X(NAME, IDX)                                                                             \
-  if (d.mechanism == IDX) {                                                                      \
-    constexpr int NV = Mech_##NAME::NS + 1;                                                      \
-    for (int part = 0; part < o->parts; part++) {                                                \
-      im.first = part == 0, im.last = part == o->parts - 1;                                      \
-      hipLaunchKernelGGL((kb_icol<Mech_##NAME>), dim3(grid.x * (FLAT / IM_CELLS)),               \
-                         dim3(Mech_##NAME::GROUPS * IM_CELLS), im_cols_lds<Mech_##NAME>, s, a, im); \
-      hipLaunchKernelGGL((kb_iwhole<Mech_##NAME>), dim3(grid.x * 2), dim3(FLAT), 0, s, a, im);   \
-      hipLaunchKernelGGL((kb_lusolve<NV>), dim3((unsigned)(cells / 64)), dim3(64), 0, s, a, im); \
-    }                                                                                            \
-    done = true;                                                                                 \
-  }
+  const auto run = [&]<class M>() {
+    if constexpr (M::NS + 1 <= IM_N) {
+      // a mechanism of more reactions than the cache has room for in the usual 64 KB
+      if constexpr (im_cols_lds<M> > 65536)
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&kb_icol<M>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)im_cols_lds<M>);
+      for (int part = 0; part < o->parts; part++) {
+        im.first = part == 0, im.last = part == o->parts - 1;
+        hipLaunchKernelGGL((kb_icol<M>), dim3(grid.x * (FLAT / IM_CELLS)), dim3(M::GROUPS * IM_CELLS), im_cols_lds<M>, s,
+                           a, im);
+        hipLaunchKernelGGL((kb_iwhole<M>), dim3(grid.x * 2), dim3(FLAT), 0, s, a, im);
+        hipLaunchKernelGGL((kb_lusolve<M::NS + 1>), dim3((unsigned)(cells / 64)), dim3(64), 0, s, a, im);
+      }
+      done = true;
+    }
+  };
+#define X(NAME, IDX) \
+  if (d.mechanism == IDX) run.template operator()<Mech_##NAME>();
   PGA_MECHANISMS(X)
 #undef X
   if (!done) {

@@ -95,18 +95,25 @@ extern "C" int32_t pga_implicit(const pga_case *c, const pga_implicit_opts *o, p
   const dim3 grid = flat_grid(a.b);
   hipStream_t s = stream_of(stream);
   bool done = false;
-#define X(NAME, IDX)                                                                              \
-  if (d.mechanism == IDX) {                                                                       \
-    constexpr int NV = Mech_##NAME::NS + 1;                                                       \
-    for (int part = 0; part < o->parts; part++) {                                                 \
-      a.first = part == 0, a.last = part == o->parts - 1;                                         \
-      hipLaunchKernelGGL((k_icol<Mech_##NAME>), dim3((unsigned)((cells + IM_CELLS - 1) / IM_CELLS)), \
-                         dim3(Mech_##NAME::GROUPS * IM_CELLS), im_cols_lds<Mech_##NAME>, s, a);   \
-      hipLaunchKernelGGL((k_iwhole<Mech_##NAME>), dim3(grid.x * 2), dim3(FLAT), 0, s, a);        \
-      hipLaunchKernelGGL((k_lusolve<NV>), dim3((unsigned)((cells + 63) / 64)), dim3(64), 0, s, a); \
-    }                                                                                             \
-    done = true;                                                                                  \
-  }
+  // a mechanism of more species than the matrices take is refused above, and its kernels are not made
+  const auto run = [&]<class M>() {
+    if constexpr (M::NS + 1 <= IM_N) {
+      // a mechanism of more reactions than the cache has room for in the usual 64 KB
+      if constexpr (im_cols_lds<M> > 65536)
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_icol<M>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)im_cols_lds<M>);
+      for (int part = 0; part < o->parts; part++) {
+        a.first = part == 0, a.last = part == o->parts - 1;
+        hipLaunchKernelGGL((k_icol<M>), dim3((unsigned)((cells + IM_CELLS - 1) / IM_CELLS)), dim3(M::GROUPS * IM_CELLS),
+                           im_cols_lds<M>, s, a);
+        hipLaunchKernelGGL((k_iwhole<M>), dim3(grid.x * 2), dim3(FLAT), 0, s, a);
+        hipLaunchKernelGGL((k_lusolve<M::NS + 1>), dim3((unsigned)((cells + 63) / 64)), dim3(64), 0, s, a);
+      }
+      done = true;
+    }
+  };
+#define X(NAME, IDX) \
+  if (d.mechanism == IDX) run.template operator()<Mech_##NAME>();
   PGA_MECHANISMS(X)
 #undef X
   if (!done) {
