@@ -328,3 +328,48 @@ def trimmed_mechanism(directory, keep=21):
         yaml.safe_dump(doc, f, sort_keys=False)
     return str(path)
 
+
+
+def mixture_of(mechanism):
+    """The mixture of a finite-rate mechanism file."""
+    from peregrine_amd.mixture import get_mixture
+
+    cfg = Config()
+    m = cfg["mixture"]
+    m["species"], m["eos"], m["T-range"], m["chemistry"] = mechanism, "tpg", (300.0, 3500.0), "finite-rate"
+    return get_mixture(cfg)
+
+
+def grown_mechanism(directory, ns, nr):
+    """A mechanism of ns species (at least nine) and nr reactions, written into directory: the H2/O2 file's
+    species with copies of them under names of their own (H2_1, ...), its reactions in turn, every second
+    round of them between the copies, each a little faster than the one it repeats."""
+    import copy
+
+    import yaml
+
+    from peregrine_amd.mixture.mixture import DATA
+
+    with open(DATA / "mechanisms" / "h2o2.yaml") as f:
+        doc = yaml.safe_load(f)
+    *active, bath = doc["species"]
+    copies = [dict(copy.deepcopy(active[m]), name=active[m]["name"] + "_1") for m in range(ns - len(active) - 1)]
+    doc["species"] = active + copies + [bath]
+    names = [s["name"] for s in doc["species"]]
+    doc["phases"][0]["species"] = names
+    base, reactions = doc["reactions"], []
+    for k in range(nr):
+        turn, m = divmod(k, len(base))
+        r = copy.deepcopy(base[m])
+        r["duplicate"] = True
+        if turn % 2:
+            r["equation"] = " ".join(t + "_1" if t + "_1" in names else t for t in r["equation"].split())
+        for key in ("rate-constant", "high-P-rate-constant"):
+            if key in r:
+                r[key]["A"] = float(r[key]["A"]) * (1.0 + 0.01 * turn)
+        reactions.append(r)
+    doc["reactions"] = reactions
+    path = Path(directory) / f"grown-{ns}-{nr}.yaml"
+    with open(path, "w") as f:
+        yaml.safe_dump(doc, f, sort_keys=False)
+    return str(path)

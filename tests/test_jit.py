@@ -94,3 +94,23 @@ def test_a_real_gas_library_at_three_species():
     assert L.pga_stage_supported(h)
     L.pga_case_destroy(h)
 
+
+
+def test_a_mechanism_of_more_species_than_the_implicit_form_takes_gets_its_library(tmp_path):
+    """Fourteen species: every source builds, and the implicit form, whose matrices take eleven, says it has
+    no work array for the case."""
+    import ctypes
+
+    mix = sp.mixture_of(sp.grown_mechanism(tmp_path, 14, 20))
+    name, records, sets, _, sig = case_mechanism(mix)
+    assert mix.ns == 14 and len(records) == 20
+    L = native.lib_at(build.build_variant(mix.ns, mechanism=(name, records, sets)))
+    desc = native.CaseDesc()
+    desc.ns, desc.eos, desc.mechanism, desc.trans = 14, 1, L.pga_mechanism_find(sig.encode()), -1
+    assert desc.mechanism == 0
+    dummy = (ctypes.c_double * 1)()
+    p, h = ctypes.cast(dummy, ctypes.c_void_p), ctypes.c_void_p()
+    assert L.pga_case_create(ctypes.byref(desc), p, p, ctypes.byref(h)) == 0
+    assert L.pga_stage_supported(h)
+    assert L.pga_implicit_worksize(h, native.box((0, 0, 0), (4, 4, 4))) == -1
+    L.pga_case_destroy(h)
