@@ -362,7 +362,7 @@ extern "C" int32_t pga_batch_create(const pga_case *c, int32_t nblocks, const pg
     for (int m = 0; m < 3; m++) {
       Box3 fb = B.b;
       (m == 0 ? fb.e0 : m == 1 ? fb.e1 : fb.e2) += 1;
-      B.t[m] = face_tiles(m, fb);
+      B.t[m] = face_tiles(m, fb, d.ns);
       slots[m] = std::max(slots[m], face_tile_slots(B.t[m]));
     }
   }

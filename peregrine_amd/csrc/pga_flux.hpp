@@ -291,8 +291,11 @@ __device__ __forceinline__ void flux_face(const double *__restrict__ K, int axis
 // side by side (an odd number of doubles, so the lanes' slots spread over every bank) and a face's four
 // cells are `step` slots apart.
 // ---------------------------------------------------------------------------
+constexpr int slot_doubles(int ns) { return (ns + 4) | 1; }
 template <int NS>
-constexpr int SLOT = (NS + 4) | 1;
+constexpr int SLOT = slot_doubles(NS);
+// the LDS a tile may take, whatever the species count: what any launch may ask for without its limit raised
+constexpr unsigned FACE_LDS = 65536;
 
 constexpr bool staged(int eos, int recon) { return recon == RECON_MUSCL && eos != EOS_REAL; }
 
@@ -324,9 +327,10 @@ __host__ inline int64_t face_tile_count(const FaceTiles &t) {
 }
 
 // The tile shape of a box's faces. i: 256 faces, fewer where short rows would bring more than 352 slots
-// (36 KB for nine species: four workgroups a CU keep their four waves a SIMD). j, k: the width whose waves
-// and staged cells cost least, a wave of faces taken as eight times its 64 lanes' staging
-__host__ inline FaceTiles face_tiles(int axis, const Box3 &b) {
+// (36 KB for nine species, 58 for the most a case may have). j, k: the width whose waves and staged cells cost
+// least, a wave of faces taken as eight times its 64 lanes' staging, among those whose slots fit FACE_LDS:
+// widths 16, 32 and 64 stage 304, 352 and 448 cells, so from 14 species on (68 KB) 64 is not taken
+__host__ inline FaceTiles face_tiles(int axis, const Box3 &b, int ns) {
   FaceTiles t{axis, 256, b, {}, {}, {}};
   if (axis == 0) {
     while (t.shape > 64 && face_tile_slots(t) > 352) t.shape /= 2;
@@ -337,6 +341,7 @@ __host__ inline FaceTiles face_tiles(int axis, const Box3 &b) {
   int64_t least = 0;
   for (int s = 4; s <= 6; s++) {
     const int64_t wi = 1 << s, ta = FLAT / wi, nbi = (b.e0 + wi - 1) / wi, full = ea / ta, rem = ea % ta;
+    if (wi * (ta + 3) * slot_doubles(ns) * (int64_t)sizeof(double) > FACE_LDS) continue;
     const int64_t waves = nbi * (full * (FLAT / 64) + (rem * wi + 63) / 64);
     const int64_t cost = waves * 64 * 8 + nbi * wi * (ea + 3 * (full + (rem > 0)));
     if (s == 4 || cost < least) least = cost, t.shape = s;

@@ -128,7 +128,7 @@ template <int NS, int EOS>
 static void launch_flux(const pga_case *c, int axis, pga_view Q, pga_view st, pga_view S, pga_view F, Box3 b,
                         hipStream_t s) {
   const int lim = c->desc.limiter, recon = c->desc.recon, prim = c->desc.primary;
-  const FaceTiles ft = face_tiles(axis, b);
+  const FaceTiles ft = face_tiles(axis, b, NS);
   const bool tiles = staged(EOS, recon);
   const dim3 grid = tiles ? dim3((unsigned)face_tile_count(ft)) : axis == 2 ? ktile_grid(b) : flat_grid(b);
   const size_t lds = tiles ? sizeof(double) * face_tile_slots(ft) * SLOT<NS> : 0;
@@ -228,7 +228,7 @@ extern "C" int32_t pga_faces(const pga_case *c, pga_view Q, pga_view state, cons
   unsigned n[3] = {0, 0, 0}, slots = 0;
   for (int axis = 0; axis < 3; axis++) {
     if (empty(boxes[axis])) continue;
-    a.t[axis] = face_tiles(axis, box3(boxes[axis]));
+    a.t[axis] = face_tiles(axis, box3(boxes[axis]), d.ns);
     if (staged(d.eos, d.recon)) {
       n[axis] = (unsigned)face_tile_count(a.t[axis]);
       slots = std::max(slots, face_tile_slots(a.t[axis]));
