@@ -410,7 +410,8 @@ typedef struct {
 } pga_implicit_opts;
 
 /* Doubles of device work pga_implicit needs for `box` (the FP64 matrices of 16-cell groups, the FP64
- * unknowns and two right-hand sides); -1 for a bad box or more than 11 species. */
+ * unknowns and two right-hand sides, and for a mechanism of some 280 reactions and more the rates' values
+ * at each cell's T); -1 for a bad box or more than 11 species. */
 int64_t pga_implicit_worksize(const pga_case *c, pga_box box);
 
 /* Implicit chemistry over the cells of `box` for a step of *dt (device): each cell integrates the

@@ -553,7 +553,7 @@ extern "C" int64_t pga_batch_implicit_worksize(const pga_batch *h) {
   if (!h || h->c->desc.ns + 1 > IM_N) return -1;
   const int64_t cells = batch_cells(h), groups = (cells + IM_G - 1) / IM_G, nv = h->c->desc.ns + 1;
   if (h->c->desc.mechanism < 0) return -1;
-  return groups * nv * nv * IM_G + 3 * nv * cells;
+  return groups * nv * nv * IM_G + (3 * nv + im_cache_work_of(h->c->desc.mechanism)) * cells;
 }
 
 extern "C" int32_t pga_batch_implicit(const pga_batch *h, const pga_implicit_opts *o, int32_t q, int32_t *sweeps,
@@ -581,18 +581,18 @@ extern "C" int32_t pga_batch_implicit(const pga_batch *h, const pga_implicit_opt
   im.begin_dQ = 0;
   im.A = work;
   im.y = im.A + groups * nv * nv * IM_G;
+  im.tc = im.y + 3 * nv * cells;
   im.ncell = cells, im.sweeps = sweeps, im.dt = dt;
   im.parts = o->parts, im.maxsweeps = o->max_sweeps, im.tol = o->tolerance;
   const BArgs a = bargs(h, q, q, 0, h->prefix[BK_CELLS]);
   const dim3 grid = tiles_grid(h->total[BK_CELLS]);
   hipStream_t s = stream_of(stream);
   bool done = false;
+  int32_t rc = PGA_OK;
   const auto run = [&]<class M>() {
     if constexpr (M::NS + 1 <= IM_N) {
-      // a mechanism of more reactions than the cache has room for in the usual 64 KB
-      if constexpr (im_cols_lds<M> > 65536)
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&kb_icol<M>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)im_cols_lds<M>);
+      done = true;
+      if ((rc = im_room<M>(reinterpret_cast<const void *>(&kb_icol<M>), "pga_batch_implicit")) != PGA_OK) return;
       for (int part = 0; part < o->parts; part++) {
         im.first = part == 0, im.last = part == o->parts - 1;
         hipLaunchKernelGGL((kb_icol<M>), dim3(grid.x * (FLAT / IM_CELLS)), dim3(M::GROUPS * IM_CELLS), im_cols_lds<M>, s,
@@ -600,7 +600,6 @@ extern "C" int32_t pga_batch_implicit(const pga_batch *h, const pga_implicit_opt
         hipLaunchKernelGGL((kb_iwhole<M>), dim3(grid.x * 2), dim3(FLAT), 0, s, a, im);
         hipLaunchKernelGGL((kb_lusolve<M::NS + 1>), dim3((unsigned)(cells / 64)), dim3(64), 0, s, a, im);
       }
-      done = true;
     }
   };
 #define X(NAME, IDX) \
@@ -611,5 +610,5 @@ extern "C" int32_t pga_batch_implicit(const pga_batch *h, const pga_implicit_opt
     set_error("pga_batch_implicit: no mechanism %d", d.mechanism);
     return PGA_EUNSUP;
   }
-  return launched("pga_batch_implicit");
+  return rc != PGA_OK ? rc : launched("pga_batch_implicit");
 }

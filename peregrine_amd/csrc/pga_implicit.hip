@@ -50,7 +50,7 @@ extern "C" int64_t pga_implicit_worksize(const pga_case *c, pga_box box) {
   if (!c || !box_ok(box) || c->desc.ns + 1 > IM_N) return -1;
   const int64_t cells = im_cells(box), groups = im_groups(cells), nv = c->desc.ns + 1;
   if (c->desc.mechanism < 0) return -1;
-  return groups * nv * nv * IM_G + 3 * nv * cells;
+  return groups * nv * nv * IM_G + (3 * nv + im_cache_work_of(c->desc.mechanism)) * cells;
 }
 
 extern "C" int32_t pga_implicit(const pga_case *c, const pga_implicit_opts *o, pga_view Q, pga_view state,
@@ -90,18 +90,18 @@ extern "C" int32_t pga_implicit(const pga_case *c, const pga_implicit_opts *o, p
   a.begin_dQ = begin_dQ != 0;
   a.A = work;
   a.y = a.A + groups * nv * nv * IM_G;
+  a.tc = a.y + 3 * nv * cells;
   a.ncell = cells, a.sweeps = sweeps, a.dt = dt, a.b = box3(box);
   a.parts = o->parts, a.maxsweeps = o->max_sweeps, a.tol = o->tolerance;
   const dim3 grid = flat_grid(a.b);
   hipStream_t s = stream_of(stream);
   bool done = false;
+  int32_t rc = PGA_OK;
   // a mechanism of more species than the matrices take is refused above, and its kernels are not made
   const auto run = [&]<class M>() {
     if constexpr (M::NS + 1 <= IM_N) {
-      // a mechanism of more reactions than the cache has room for in the usual 64 KB
-      if constexpr (im_cols_lds<M> > 65536)
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_icol<M>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)im_cols_lds<M>);
+      done = true;
+      if ((rc = im_room<M>(reinterpret_cast<const void *>(&k_icol<M>), "pga_implicit")) != PGA_OK) return;
       for (int part = 0; part < o->parts; part++) {
         a.first = part == 0, a.last = part == o->parts - 1;
         hipLaunchKernelGGL((k_icol<M>), dim3((unsigned)((cells + IM_CELLS - 1) / IM_CELLS)), dim3(M::GROUPS * IM_CELLS),
@@ -109,7 +109,6 @@ extern "C" int32_t pga_implicit(const pga_case *c, const pga_implicit_opts *o, p
         hipLaunchKernelGGL((k_iwhole<M>), dim3(grid.x * 2), dim3(FLAT), 0, s, a);
         hipLaunchKernelGGL((k_lusolve<M::NS + 1>), dim3((unsigned)((cells + 63) / 64)), dim3(64), 0, s, a);
       }
-      done = true;
     }
   };
 #define X(NAME, IDX) \
@@ -120,7 +119,7 @@ extern "C" int32_t pga_implicit(const pga_case *c, const pga_implicit_opts *o, p
     set_error("pga_implicit: no mechanism %d", d.mechanism);
     return PGA_EUNSUP;
   }
-  return launched("pga_implicit");
+  return rc != PGA_OK ? rc : launched("pga_implicit");
 }
 
 extern "C" int64_t pga_lu_worksize(int64_t n, int32_t nv) {

@@ -26,7 +26,8 @@
 //
 // The implicit form's work array holds the FP64 matrices, [group of 16 cells][(ns + 1)^2 entries]
 // [16 cells] (a row of the 16 cells' same entry is 128 contiguous bytes, so the lane-per-cell
-// kernels move whole segments), then y, f at y's FP32 rounding and f at y, [ns + 1][cells] doubles each.
+// kernels move whole segments), then y, f at y's FP32 rounding and f at y, [ns + 1][cells] doubles each, then
+// the caches of a mechanism too large for LDS (im_cache_work).
 // The FP32 factors never leave the registers of the solve. The batched solve of caller-given systems
 // keeps its FP32 factors in a work array the same way, [group][144 entries][16 cells].
 #pragma once
@@ -35,6 +36,7 @@
 
 #include "generated/mechanisms.hpp"
 #include "pga_chem.hpp"
+#include "pga_internal.hpp"
 
 namespace pga {
 
@@ -164,6 +166,7 @@ struct ImArgs {
   int begin_dQ, first, last;
   double *A;     // the FP64 matrices, group-major with nv^2 entries
   double *y;     // [ns + 1][ncell] three times: the part's start (then its end), f at its FP32 rounding, f at it
+  double *tc;    // [im_cache_work][ncell]: the caches of a mechanism whose workgroups' caches pass LDS
   int64_t ncell;
   int32_t *sweeps;
   const double *dt;
@@ -298,10 +301,42 @@ __device__ __forceinline__ int refine(const float *__restrict__ W, const double 
 // two launches take 97 + 69 us for the 64^3 cells in place of 260, at three waves a SIMD. The 64^3 step went
 // from 1.45 to 1.16 ms, that of 16 boxes of 3.0 million cells in all from 16.9 to 13.0 ms.
 
-constexpr int IM_CELLS = 64;  // cells of a workgroup of the species columns
+// A workgroup's caches pass gfx950's 160 KB of LDS from 320 values a cell on, some 280 reactions of nine
+// species: such a mechanism's go through the work array, the same code and values (the start of a part stores
+// them, its columns read them back through L2).
 
+constexpr int IM_CELLS = 64;  // cells of a workgroup of the species columns
+constexpr size_t IM_LDS = 163840;
+
+// the doubles of the work array a cell's cache takes, and the LDS of a workgroup's
 template <class M>
-constexpr size_t im_cols_lds = sizeof(double) * im_cache_n<M> * IM_CELLS;
+constexpr int im_cache_work = sizeof(double) * im_cache_n<M> * IM_CELLS > IM_LDS ? im_cache_n<M> : 0;
+template <class M>
+constexpr size_t im_cols_lds = im_cache_work<M> ? 0 : sizeof(double) * im_cache_n<M> * IM_CELLS;
+
+// im_cache_work of the library's mechanism of that number
+inline int im_cache_work_of(int mechanism) {
+  int n = 0;
+#define X(NAME, IDX) \
+  if (mechanism == IDX) n = im_cache_work<Mech_##NAME>;
+  PGA_MECHANISMS(X)
+#undef X
+  return n;
+}
+
+// lets a kernel of the columns be launched with its LDS where that passes the 64 KB any launch may ask for
+template <class M>
+inline int32_t im_room(const void *kernel, const char *who) {
+  if constexpr (im_cols_lds<M> > 65536) {
+    const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)im_cols_lds<M>);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      set_error("%s: %d bytes of LDS a workgroup: %s", who, (int)im_cols_lds<M>, hipGetErrorString(e));
+      return PGA_EHIP;
+    }
+  }
+  return PGA_OK;
+}
 
 // the y of a cell at the part's start: the first part's from Q and the state, a later one's as the last part
 // left it (selected rather than branched, one copy of the code)
@@ -318,17 +353,31 @@ __device__ __forceinline__ void im_y0(const ImArgs &a, const View &Q, const View
 
 // a wave's view of the constants and of its lane's place in the cache, as values the compiler cannot match
 // with another group's: it would read what the groups share ahead of the branch that tells them apart, and
-// hold it in registers 
+// hold it in registers
+template <bool WORK>
 struct ImGroup {
   Constants K, C;
   double *lds;
   unsigned lane;
-  __device__ __forceinline__ ImGroup(const ImArgs &a, double *l) : K(constants(a.K)), C(constants(a.C)), lds(l) {
+  __device__ __forceinline__ ImGroup(const ImArgs &a, double *l, int64_t) : K(constants(a.K)), C(constants(a.C)), lds(l) {
     lane = threadIdx.x % IM_CELLS;
     asm volatile("" : "+s"(K), "+s"(C), "+v"(lane));
   }
   // entry e of the lane's cell
   __device__ __forceinline__ double &operator()(int e) const { return lds[e * IM_CELLS + lane]; }
+};
+
+// the same of a cache in the work array
+template <>
+struct ImGroup<true> {
+  Constants K, C;
+  double *tc;
+  int64_t nc;
+  __device__ __forceinline__ ImGroup(const ImArgs &a, double *, int64_t code)
+      : K(constants(a.K)), C(constants(a.C)), tc(a.tc + code), nc(a.ncell) {
+    asm volatile("" : "+s"(K), "+s"(C), "+v"(tc));
+  }
+  __device__ __forceinline__ double &operator()(int e) const { return tc[e * nc]; }
 };
 
 // ends a group's branch: without it the stores that end every branch are made one store where they join,
@@ -337,10 +386,10 @@ __device__ __forceinline__ void im_branch_end() { asm volatile(""); }
 
 // group G's share of a cell's cache at T
 template <class M, int G>
-__device__ __forceinline__ void ijac_part(const ImArgs &a, double T, double *lds) {
+__device__ __forceinline__ void ijac_part(const ImArgs &a, double T, double *lds, int64_t code) {
 #pragma clang fp contract(off)
   constexpr int NS = M::NS, NT = sizeof(typename M::TCache) / sizeof(double);
-  const ImGroup X(a, lds);
+  const ImGroup<(im_cache_work<M> > 0)> X(a, lds, code);
   const Gas<NS> g{X.K};
   const auto put = [&](int e, double v) { X(e) = v; };
   M::template tstate_part<G>(g, X.C, T, put);
@@ -361,7 +410,7 @@ __device__ __forceinline__ void ijac_group(const ImArgs &a, double rho, double r
 #pragma clang fp contract(off)
   constexpr int NS = M::NS, NV = NS + 1, NT = sizeof(typename M::TCache) / sizeof(double);
   constexpr int m0 = G * M::COLS, nm = NS - m0 < M::COLS ? NS - m0 : M::COLS;
-  const ImGroup X(a, lds);
+  const ImGroup<(im_cache_work<M> > 0)> X(a, lds, code);
   double Yp[M::COLS] = {}, hd[M::COLS] = {}, omega[M::COLS + 1][NS];
   const double h = *a.dt / a.parts;
 #pragma unroll
@@ -432,7 +481,7 @@ __device__ __forceinline__ void ijac_columns(const ImArgs &a, const View &Q, con
     for (int r = 0; r < NV; r++) a.y[r * a.ncell + code] = y0[r];
   }
   const double T = (double)(float)y0[NS];
-  im_group<M::GROUPS>(wave, [&]<int G>() { ijac_part<M, G>(a, T, lds); });
+  im_group<M::GROUPS>(wave, [&]<int G>() { ijac_part<M, G>(a, T, lds, code); });
   __syncthreads();
 #pragma unroll
   for (int n = 0; n < NS; n++) Y[n] = (double)(float)y0[n];

@@ -373,3 +373,28 @@ def grown_mechanism(directory, ns, nr):
     with open(path, "w") as f:
         yaml.safe_dump(doc, f, sort_keys=False)
     return str(path)
+
+
+# reactions whose caches pass 64 KB of LDS for the implicit form's 64 cells a workgroup, and all of it (160 KB)
+CACHE_PAST_64K, CACHE_PAST_LDS = 115, 310
+
+
+def recombination_mechanism(directory, nr):
+    """Oxygen atoms and molecules in nitrogen by nr reactions, written into directory: 2 O + M <=> O2 + M and
+    2 O + O2 <=> 2 O2 in turn, each a little faster than the last: few species, as many reactions as asked."""
+    import yaml
+
+    from peregrine_amd.mixture.mixture import DATA
+
+    with open(DATA / "mechanisms" / "h2o2.yaml") as f:
+        doc = yaml.safe_load(f)
+    doc["species"] = [s for s in doc["species"] if s["name"] in ("O", "O2", "N2")]
+    doc["phases"][0]["species"], doc["phases"][0]["elements"] = [s["name"] for s in doc["species"]], ["O", "N"]
+    doc["reactions"] = [
+        {"equation": "2 O + M <=> O2 + M" if k % 2 == 0 else "2 O + O2 <=> 2 O2", "duplicate": True,
+         "rate-constant": {"A": 1.2e15 * (1.0 + 0.01 * k), "b": -1.0 + 0.001 * k, "Ea": 10.0 * k},
+         **({"type": "three-body", "efficiencies": {"O2": 0.5}} if k % 2 == 0 else {})} for k in range(nr)]
+    path = Path(directory) / f"recombination-{nr}.yaml"
+    with open(path, "w") as f:
+        yaml.safe_dump(doc, f, sort_keys=False)
+    return str(path)

@@ -4,6 +4,8 @@ own, keyed by the sha256 of what it is compiled from, as the reference keys its 
 (peregrine/backend/base/compiler.py:42-64). These tests build the two libraries the device tests
 use, so those find them cached."""
 
+import pytest
+
 import support as sp
 from peregrine_amd import build, native
 from peregrine_amd.config import Config
@@ -113,4 +115,25 @@ def test_a_mechanism_of_more_species_than_the_implicit_form_takes_gets_its_libra
     assert L.pga_case_create(ctypes.byref(desc), p, p, ctypes.byref(h)) == 0
     assert L.pga_stage_supported(h)
     assert L.pga_implicit_worksize(h, native.box((0, 0, 0), (4, 4, 4))) == -1
+    L.pga_case_destroy(h)
+
+
+@pytest.mark.parametrize("nr", [sp.CACHE_PAST_64K, sp.CACHE_PAST_LDS])
+def test_a_mechanism_of_many_reactions_gets_its_library(tmp_path, nr):
+    """The implicit form takes a mechanism however large its caches are: past a workgroup's LDS they go in the
+    work array, which is as much larger."""
+    import ctypes
+
+    mix = sp.mixture_of(sp.recombination_mechanism(tmp_path, nr))
+    name, records, sets, _, sig = case_mechanism(mix)
+    assert mix.ns == 3 and len(records) == nr
+    L = native.lib_at(build.build_variant(mix.ns, mechanism=(name, records, sets)))
+    desc = native.CaseDesc()
+    desc.ns, desc.eos, desc.mechanism, desc.trans = 3, 1, L.pga_mechanism_find(sig.encode()), -1
+    dummy = (ctypes.c_double * 1)()
+    p, h = ctypes.cast(dummy, ctypes.c_void_p), ctypes.c_void_p()
+    assert L.pga_case_create(ctypes.byref(desc), p, p, ctypes.byref(h)) == 0
+    # 16 cells: their 4 x 4 matrices, y and two of f, and per cell the cache where it does not fit
+    size = L.pga_implicit_worksize(h, native.box((0, 0, 0), (16, 1, 1))) / 16.0 - 16 - 3 * 4
+    assert size == 0 if nr == sp.CACHE_PAST_64K else size > 320
     L.pga_case_destroy(h)
