@@ -33,18 +33,6 @@ __global__ __launch_bounds__(WT) void k_stage(StageArgs a) {
   stage_cells<NE, CHEM>(a, i, j, kbeg, min(kbeg + a.kc, a.s2 + a.n2), lbeg, min(lbeg + a.rows, NE));
 }
 
-// The row groups a block's stage goes in. A thread waits on memory once a row: a block too small to fill the
-// SIMDs waits for its rows one after another, so below 2^17 cells (two waves to each of the 1024 SIMDs) it takes
-// them by several threads, as many as bring eight waves to each (the rows need nothing of each other but 1/J).
-// Nine species: 25 to 20 us a launch at 61 x 47 x 33, the 50 x 37 x 45
-// sub-stepped step from 278 to 260; the 215 040 cells of 80 x 48 x 56 take 41.8 us whole and 44.2 in three groups
-static void row_groups(StageArgs &a, int ne) {
-  const int64_t cells = std::max<int64_t>(1, (int64_t)a.n0 * a.n1 * a.n2);
-  const int64_t want = cells > (int64_t(1) << 17) ? 1 : std::min<int64_t>(ne, (int64_t(8) * 1024 * 64 + cells - 1) / cells);
-  a.rows = (ne + (int)want - 1) / (int)want;
-  a.groups = (ne + a.rows - 1) / a.rows;
-}
-
 // a small block's stage and the EOS of its result in one launch, for a few rows: each cell's reads at once, its
 // EOS from the new Q in registers (a block of a few thousand cells is bound by launches and waits)
 template <int NS, int EOS, bool CHEM>
@@ -213,7 +201,7 @@ static int32_t stage_impl(const char *who, const pga_case *c, pga_view Qin, pga_
   const Box3 b = box3(box);
   // a block of at most 2^16 cells (up to 40^3) whose rows fit registers in one launch, any other in two
   const bool whole = (int64_t)a.n0 * a.n1 * a.n2 <= (int64_t(1) << 16);
-  row_groups(a, ne);
+  row_groups(a, ne, grid.z);
   const dim3 rgrid(grid.x, grid.y, grid.z * a.groups);
   const bool done = dispatch_eos(d, [&]<int N, int E>() {
     if constexpr (N + 4 <= 8) {

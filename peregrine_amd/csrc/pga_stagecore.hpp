@@ -158,6 +158,20 @@ __device__ __forceinline__ void stage_cell_regs(const StageArgs &a, int i, int j
   }
 }
 
+// The row groups a block's stage goes in. A thread waits on memory once a row: a block too small to fill the
+// SIMDs waits for its rows one after another, so below 2^17 cells (two waves to each of the 1024 SIMDs) it takes
+// them by several threads, as many as bring eight waves to each (the rows need nothing of each other but 1/J).
+// Nine species: 25 to 20 us a launch at 61 x 47 x 33, the 50 x 37 x 45 sub-stepped step from 278 to 260; the
+// 215 040 cells of 80 x 48 x 56 take 41.8 us whole and 44.2 in three groups. The groups share the grid's z with
+// the planes, of which a box has up to the 65 535 z may have: a line of so many cells along k takes fewer
+__host__ inline void row_groups(StageArgs &a, int ne, unsigned planes) {
+  const int64_t cells = std::max<int64_t>(1, (int64_t)a.n0 * a.n1 * a.n2);
+  int64_t want = cells > (int64_t(1) << 17) ? 1 : std::min<int64_t>(ne, (int64_t(8) * 1024 * 64 + cells - 1) / cells);
+  want = std::max<int64_t>(1, std::min<int64_t>(want, 65535 / planes));
+  a.rows = (ne + (int)want - 1) / (int)want;
+  a.groups = (ne + a.rows - 1) / a.rows;
+}
+
 // The divergence, the source and the RK combine of rows lbeg..lend-1 of the cells (i, j, kbeg..kend-1) of one
 // column: memory-bound. A row at a time in a rolled loop keeps ~30 registers, so eight waves per SIMD hide
 // the loads' latency
