@@ -61,12 +61,19 @@ __global__ __launch_bounds__(256) void k_stage_eos(const double *__restrict__ K,
   eos_cell<NS, EOS>(K, Q, stin, stout, i, j, k);
 }
 
-// the carried species' production rates of each cell (chemint/kernels/cell.mako:5-20), the
-// source a reacting stage begins dQ with. Five waves a SIMD: left to itself the compiler takes four (110
-// registers), at 128^3 in 159 us where five take 150
+// The waves a SIMD the rates are held to. Nine species and fewer: left to itself the compiler takes four (110
+// registers), at 128^3 in 159 us where five take 150; with 60 reactions, 419 us a step at 64^3 by five and 422
+// by its own choice. More species would spill at five (16 with 68 reactions: 50 registers) and are left to it:
+// the 64^3 step of 10 species and 40 reactions takes 386 us where five waves took 404, of 11 and 40 412 against
+// 423, of 16 and 68 601 against 612, its 96^3 step 1805 against 1921
 template <class M>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_rates(const double *__restrict__ K, const double *__restrict__ C, View Q,
-                                               View st, View rates, Box3 b) {
+constexpr int rates_waves = M::NS <= 9 ? 5 : 1;
+
+// the carried species' production rates of each cell (chemint/kernels/cell.mako:5-20), the
+// source a reacting stage begins dQ with
+template <class M>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(rates_waves<M>))) void k_rates(
+    const double *__restrict__ K, const double *__restrict__ C, View Q, View st, View rates, Box3 b) {
   int i, j, k;
   if (!cell_of(b, i, j, k)) return;
   rates_cell<M>(K, C, Q, st, rates, i, j, k);
@@ -116,10 +123,8 @@ __global__ __launch_bounds__(256) void k_halo(HaloArgs a) {
 // 128^3 where the two launches took 150 + 30, 21 where they took 19 + 10 at 61 x 47 x 33. (The rates among the
 // faces' workgroups instead held them to the faces' three waves a SIMD: 596 us against 371 + 155.)
 template <class M>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_halo_rates(HaloArgs a, unsigned halo,
-                                                                                           const double *__restrict__ C,
-                                                                                           View Q, View st, View rates,
-                                                                                           Box3 b) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(rates_waves<M>))) void k_halo_rates(
+    HaloArgs a, unsigned halo, const double *__restrict__ C, View Q, View st, View rates, Box3 b) {
   if (blockIdx.x < halo) {
     halo_block<M::NS, EOS_TPG>(a, blockIdx.x);
     return;
