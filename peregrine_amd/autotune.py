@@ -2,8 +2,9 @@
 
 A batch's blocks fall in size classes by their interior's extent along i (the contiguous index a
 tile's lanes run along). Per class, the autotuner times the stage's divergence-and-combine launch
-with each candidate column tile (width along i and k-planes per thread) and the k-sweep with each
-candidate tile width, holding the other classes at their current choice, and keeps the fastest. A
+with each candidate column tile (width along i and k-planes per thread) and, for a scheme that has the
+choice (``trials``), the k-sweep with each candidate tile width, holding the other classes at their
+current choice, and keeps the fastest. A
 block-at-a-time launch takes 64-wide tiles: on a 16-cell-wide block three quarters of their lanes
 would idle. The choice changes only the speed: a cell's arithmetic is the same in every tile.
 
@@ -21,6 +22,7 @@ import os
 from pathlib import Path
 
 from peregrine_amd import native
+from peregrine_amd.simulator import EOS, RECON
 
 # size classes by interior cells along i: (name, upper bound inclusive)
 CLASSES = (("narrow", 24), ("small", 48), ("medium", 80), ("wide", 1 << 30))
@@ -70,6 +72,16 @@ def _time(solver, launch, reps=5):
     return e0.elapsed_time(e1) / reps
 
 
+def trials(desc):
+    """The kinds of launch whose tiles the case has a choice of, each with its candidates. The k sweep's
+    width is read only where the faces' stencils come from the cell arrays (the constant reconstruction,
+    the cubic gas): other MUSCL faces go in staged tiles, which the library shapes by the box."""
+    kinds = [("stage", STAGE_TILES)]
+    if desc.recon != RECON["muscl"] or desc.eos == EOS["real-gas"]:
+        kinds.append(("fluxk", FLUXK_TILES))
+    return kinds
+
+
 def tune(solver):
     """{class: {"stage": (wi, kc), "fluxk": ki}} for the solver's blocks: from the cache, or timed now.
     Timing runs the stage into the unused derivative register with a scratch copy of each block's
@@ -107,7 +119,7 @@ def tune(solver):
             batch.close()
 
     for c in sorted(census):
-        for kind, cands in (("stage", STAGE_TILES), ("fluxk", FLUXK_TILES)):
+        for kind, cands in trials(solver.case.desc):
             best = None
             for cand in cands:
                 trial = {k: dict(v) for k, v in choice.items()}
