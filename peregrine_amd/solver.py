@@ -500,11 +500,13 @@ class Solver:
             self._exchange(lambda b: b.grads, 3 * self.sim.ngrad, 1, 0, 1)
 
     def _gradient_slabs(self, blk, turned):
-        """The halo slabs that mirror a block's cells, as pga_transport_grads_slabs takes them."""
+        """The halo slabs that mirror a block's cells, as pga_transport_grads_slabs takes them: those of the
+        interfaces that meet its own back."""
         slabs = []
-        for dst in self.blocks if not turned else ():
-            slabs += [(dst.grads.view(), placement(dst, f, blk, 1)) for f in dst.faces.values()
-                      if f.nbr is not None and self.blocks[f.nbr] is blk]
+        for f in blk.faces.values():
+            if f.nbr is not None and not turned:
+                nbr = self.blocks[f.nbr]
+                slabs.append((nbr.grads.view(), placement(nbr, nbr.faces[f.nbrnface], blk, 1)))
         n = len(slabs)
         return (n, (native.View * n)(*[v for v, _ in slabs]),
                 *(native.ints([x for _, p in slabs for x in p[m]]) for m in range(4)))
