@@ -190,8 +190,9 @@ def render(name, records, sets, ns):
         at += 2 + ns
     off["gRT"] = at
     off["kx"] = at + ns
-    _tstate_part(w, L, records, ns, off, logform, product)
-    _fold_columns(w, L, records, sets, ns, off, logform, product)
+    if ns <= IMPLICIT_NS:
+        _tstate_part(w, L, records, ns, off, logform, product)
+        _fold_columns(w, L, records, sets, ns, off, logform, product)
     w("  __device__ __forceinline__ static void production(const Gas<NS> &g, Constants C,")
     w("                                                    double rho, const double (&Y)[NS], double T, double (&omega)[NS]) {")
     w("    Rates s;")
@@ -381,6 +382,9 @@ class _ColumnNames(_Names):
 
 # the species columns a lane takes beside the base (implicit chemistry's workgroups have a wave a group)
 COLUMNS = 3
+# the species whose matrices implicit chemistry takes (IM_N less T, pga_implicit.hpp): a mechanism of more has
+# no columns
+IMPLICIT_NS = 11
 
 
 def _touches(r, sp):
@@ -445,7 +449,7 @@ def _tstate_part(w, L, records, ns, off, logform, product):
 
 def _fold_columns(w, L, records, sets, ns, off, logform, product):
     """The rates at one T of a base composition, omega[0], and with one species moved for each of a group's
-    COLUMNS species: cstate + fold_cached's values of each, a reaction's rate evaluated again only for the
+    COLUMNS species: ratestate + fold's values of each, a reaction's rate evaluated again only for the
     columns whose species it reads."""
     w("  template <int G, class TC>")
     w("  __device__ __forceinline__ static void fold_columns(Constants K, Constants C, double rho,")

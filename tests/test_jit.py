@@ -137,3 +137,12 @@ def test_a_mechanism_of_many_reactions_gets_its_library(tmp_path, nr):
     size = L.pga_implicit_worksize(h, native.box((0, 0, 0), (16, 1, 1))) / 16.0 - 16 - 3 * 4
     assert size == 0 if nr == sp.CACHE_PAST_64K else size > 320
     L.pga_case_destroy(h)
+
+
+@pytest.mark.parametrize("ns", [9, 11, 12, 14])
+def test_only_a_mechanism_the_implicit_form_takes_has_its_columns(tmp_path, ns):
+    mix = sp.mixture_of(sp.grown_mechanism(tmp_path, ns, 20))
+    name, records, sets, _, _ = case_mechanism(mix)
+    text = build.mechanism_texts([(name, records, sets, ns)])[f"mech_{name}.hpp"]
+    assert ("fold_columns" in text) == ("tstate_part(" in text) == (ns <= 11)
+    assert "struct TCache" in text
