@@ -450,7 +450,8 @@ int32_t pga_lu_solve(int64_t n, int32_t nv, const double *A, const double *b, do
  * batch, read from slab_from[t] with orientation digits slab_orient[t] (1 2 3 aligned). Tile shapes
  * (0 for the defaults): stage_wi the stage's tile width along i (16, 32 or 64; its tiles are
  * stage_wi x 256 / stage_wi columns), stage_kc the k-planes a stage thread walks, flux_ki the k-sweep's
- * tile width along i (16, 32 or 64; 256 / flux_ki faces along k). */
+ * tile width along i (16, 32 or 64; 256 / flux_ki faces along k; not read by MUSCL on an ideal gas, whose
+ * faces go in tiles of the library's choice). */
 typedef struct {
   pga_view Q[4];
   pga_view state, iS, jS, kS, iF, jF, kF, detJinv, rates;

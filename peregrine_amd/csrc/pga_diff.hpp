@@ -7,10 +7,11 @@
 // compiler's schedule puts each load just ahead of its use, twenty and more waits a face at the registers
 // of one row, so the reads are made in groups that end in a scheduling barrier: the rows of the velocity
 // and T, then the species' two at a time (four at a time is no faster). The arrays share their layout, and
-// a cell's reads go through View::run: each array's plane is a scalar base, the cell one vector offset. A
-// Taylor-Green box's faces went from 14.9 to 11.4 us a launch at 32^3 and from 38.8 to 34.9 us at 57^3, the
-// step of the 256 x 128 x 64 real-gas layer from 3.59 to 3.47 ms; nine species with MUSCL take as long as
-// before (110 us at 80 x 48 x 56).
+// a cell's reads go through View::run: each array's plane is a scalar base, the cell one vector offset. With
+// the advective flux as it stands, a Taylor-Green box's faces take 11.6 us a launch at 32^3 and 34.5 at 57^3 so,
+// 14.9 and 38.8 with the reads left to the schedule (the faces of an earlier advective flux, whose schedule
+// happened to be kinder, took 11.0 and 35.4: at 32^3 the groups only win that back); the step of the 256 x
+// 128 x 64 real-gas layer 3.47 ms against 3.59; nine species with MUSCL as long either way (110 us at 80 x 48 x 56).
 #pragma once
 
 #include "pga_common.hpp"

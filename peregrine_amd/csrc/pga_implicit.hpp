@@ -301,9 +301,8 @@ __device__ __forceinline__ int refine(const float *__restrict__ W, const double 
 // two launches take 97 + 69 us for the 64^3 cells in place of 260, at three waves a SIMD. The 64^3 step went
 // from 1.45 to 1.16 ms, that of 16 boxes of 3.0 million cells in all from 16.9 to 13.0 ms.
 
-// A workgroup's caches pass gfx950's 160 KB of LDS from 320 values a cell on, some 280 reactions of nine
-// species: such a mechanism's go through the work array, the same code and values (the start of a part stores
-// them, its columns read them back through L2).
+// A workgroup's caches pass gfx950's 160 KB of LDS from 321 values a cell on, some 280 reactions of nine
+// species: such a mechanism's go through the work array, the same code and values.
 
 constexpr int IM_CELLS = 64;  // cells of a workgroup of the species columns
 constexpr size_t IM_LDS = 163840;

@@ -1,11 +1,10 @@
-// The fused RK stage: after a stage's three flux sweeps (pga_flux, one face per lane), one pass
-// over the block's interior does what the reference does in three more launches per stage
+// The fused RK stage: after a stage's faces (pga_faces), one pass over the block's interior does what the reference does in three more launches per stage
 // (divergence, combine, interior EOS; simulator/advec/simulator.py:57-87,
 // integrators/rungekutta.py:33-39) with the chemistry source added on the way; and the halo pass
 // before the sweeps (exchange of Q and the EOS over the halo slabs) is one launch.
 //
-// A reacting case takes its source from pga_rates, launched before the stage: the production
-// rates need ~100 registers of their own.
+// A reacting case takes its source from pga_rates or, with the halo pass in the same launch,
+// pga_halo_rates, before the faces: the production rates need ~100 registers of their own.
 //
 // Each thread owns one (i, j) column of cells and walks a chunk of k-planes. Per cell it sums its
 // six face fluxes in the reference's order, adds the chemistry source, takes the RK combine,

@@ -877,9 +877,11 @@ class Solver:
         return stage_slabs(blk.ncell[2], int(self.cfg["backend-mi355x"]["stage-slabs"]))
 
     def _fused_step(self):
-        """A step by stages of five launches per block: the halo pass (exchange and halo EOS, unless
-        from_prims left the halos ready), the chemistry rates, the three flux sweeps, and the fused
-        divergence + source + combine + EOS, in place on the reference's stage registers."""
+        """A step by stages, per block: the halo pass (exchange and halo EOS, with the coupled rates in the
+        same launch) and the walls' halos, unless from_prims left the halos ready; a viscous case's
+        transport and gradients; the rates not yet taken; every axis's faces in one launch and the walls'
+        fluxes; and the fused divergence + source + combine + EOS, in place on the reference's stage
+        registers."""
         kc = int(self.cfg["backend-mi355x"]["k-chunk"])
         for n, regs in enumerate(self.integ.stageregs(self.regs)):
             mixed = False
