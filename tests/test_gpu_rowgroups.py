@@ -6,6 +6,7 @@ import pytest
 
 import support as sp
 from peregrine_amd import get_backend, get_solver, mesher
+from test_gpu_parity import _rowerr, _run_pair
 
 pytestmark = pytest.mark.gpu
 
@@ -25,3 +26,15 @@ def test_a_stage_by_row_groups_is_the_sequence(gpu, n):
         out.append((blk.Q.get()[blk.interior], blk.state.get()[blk.interior]))
     for got, want in zip(*out):
         np.testing.assert_array_equal(got, want)
+
+
+def test_a_long_line_along_k_steps_as_the_oracle(gpu):
+    """Nine species on 5100 cells one to a plane, whose thirteen rows in groups of their own would take more of
+    the grid's z than a box's planes may: the walled line by the fused stage, within the reacting case's bound."""
+    L = (0.01, 0.01, 0.4)
+    mb, hb = _run_pair("h2o2", "muscl", "hllc", "koren", True, "tvd-rk3", (1, 1, 5100), 3, 1e-9,
+                       lambda x: sp.reacting_flow(x, 1, L), L, walls=range(6))
+    assert mb.fused
+    g = hb.ng
+    got = mb.blocks[0].Q.get()[g:-g, g:-g, g:-g].transpose(3, 2, 1, 0)
+    assert _rowerr(got, hb.regs[0][hb.interior()]) < 1e-10
